@@ -99,6 +99,10 @@ namespace imh {
 // block is replaced, not freed: graphs captured earlier may still address it.
 int stream_scratch(imh_stream *s, int slot, size_t bytes, void **out);
 
+// The same where the caller can do without: false, with no error set, when the
+// slot would have to grow while the stream captures or memory is short.
+bool stream_scratch_optional(imh_stream *s, int slot, size_t bytes, void **out);
+
 // Make the stream's device current for the calling thread.
 int use_device(const imh_device *dev);
 

@@ -23,6 +23,11 @@ size_t gemm_workspace_bytes(int M, int N, int K, int nmat, int cus);
 int encode_gemm(imh_stream *s, const __half *x, int M, const imh_affine_int4_weight *w0,
                 const imh_affine_int4_weight *w1, int epi, __half *y0, __half *y1, void *workspace);
 
+// The same with INT8 weights (one matrix, plain store).  *used false: nothing
+// was launched, as the stream's scratch cannot hold the operand planes (a
+// capture, or no memory): the caller's scratch-free path runs.
+int encode_gemm_int8(imh_stream *s, const __half *x, int M, const imh_affine_int8_weight *w, __half *y, bool *used);
+
 // Sum of squares of a 256-thread workgroup's per-thread partials, in the
 // order of a halving tree over red[] (t + 128, then + 64, ... + 1): wave 0
 // forms the first two levels from red[], shuffles do the rest.  Two barriers

@@ -63,6 +63,14 @@ int stream_scratch(imh_stream *s, int slot, size_t bytes, void **out) {
     return IMH_OK;
 }
 
+bool stream_scratch_optional(imh_stream *s, int slot, size_t bytes, void **out) {
+    if (s->capturing && s->scratch_bytes[slot] < bytes) return false;
+    if (stream_scratch(s, slot, bytes, out) == IMH_OK) return true;
+    (void)hipGetLastError();   // the failed allocation is not the next launch's error
+    clear_error();
+    return false;
+}
+
 }  // namespace imh
 
 // Byte fill used by imh_fill_zero: 16-byte stores for the aligned body.

@@ -189,3 +189,50 @@ def test_gemm_fused_residual_norm(dev, stream, m, n, k):
     assert_close(y.read(), y_ref, what="gemm resnorm y", ulps=ulps_for(True))
     assert np.array_equal(res.read().view(np.uint16), res_ref.view(np.uint16))
     assert_close(nrm.read(), nrm_ref.astype(np.float32), rel=1e-3, max_abs=2e-3, what="gemm normed")
+
+
+@pytest.mark.parametrize("m,n,k,awq", [
+    (32, 256, 128, True),      # one group, the smallest tile, one column tile
+    (33, 257, 1152, True),     # one row into a second tile half, one column past a tile, odd group count
+    (65, 513, 1152, False),    # without AWQ: the activation straight from x, constants read in place
+    (130, 31, 256, False),     # fewer columns than one fragment
+])
+def test_gemm_tile_edges(dev, stream, m, n, k, awq):
+    """The GEMM at the edges of its tiles against the exact value of the uploaded weights
+    (f64): one f16 step plus 2^-16 of the summed magnitudes (the f32 sums, and x / awq's ~22 bits)."""
+    w, s = weight(n, k, m + n, awq)
+    q = quant.quantize_int4(w, awq_scales=s)
+    x16 = acts(m, k, 3 * m + k)
+    xd, yd = dev.upload(x16), dev.empty((m, n), np.float16)
+    ops.encode_projection(stream, xd, ops.AffineQuantizedWeight(dev, q), yd, m)
+    stream.sync()
+    a = x16.astype(np.float64) if s is None else x16.astype(np.float64) / s.astype(np.float16).astype(np.float64)
+    W = exact_weights(q)
+    exact = a @ W.T
+    bound = np.spacing(np.abs(exact).astype(np.float16)).astype(np.float64) + 2.0 ** -16 * (np.abs(a) @ np.abs(W).T)
+    err = np.abs(yd.read().astype(np.float64) - exact)
+    assert np.all(err <= bound), f"m={m} n={n} k={k} awq={awq}: worst {np.max(err / bound):.2f} of the bound"
+
+
+def test_gemm_capture_reads_constants_in_place(dev):
+    """Under capture with scratch for the activation planes only, the GEMM reads scales and
+    zero-points in place: the replays equal the eager result bit for bit."""
+    m, k = 1024, 2048     # planes: 8 MiB, the first call's scratch with its constants just above
+    w, s = weight(256, k, 91, True)
+    small = ops.AffineQuantizedWeight(dev, quant.quantize_int4(w, awq_scales=s))
+    w2, _ = weight(8192, k, 92, False)
+    wide = ops.AffineQuantizedWeight(dev, quant.quantize_int4(w2, awq_scales=s))
+    x16 = acts(m, k, 93)
+    st = dev.stream()
+    xd, y0 = dev.upload(x16), dev.empty((m, 256), np.float16)
+    ye, yg = dev.empty((m, 8192), np.float16), dev.empty((m, 8192), np.float16)
+    ops.encode_projection(st, xd, small, y0, m)
+    g = st.capture(lambda: ops.encode_projection(st, xd, wide, yg, m))
+    ops.encode_projection(st, xd, wide, ye, m)
+    st.sync()
+    want = ye.read().view(np.uint16)
+    for _ in range(2):
+        st.zero(yg)
+        g.launch()
+        st.sync()
+        assert np.array_equal(yg.read().view(np.uint16), want)

@@ -84,6 +84,42 @@ def test_int8_projection(dev, stream, n, k, b, awq):
     assert rel_l2(got, ref) <= 1e-3
 
 
+@pytest.mark.parametrize("n,k,b,awq", [
+    (256, 128, 13, False),     # GEMM: one group, one plane, one 32-row tile
+    (1000, 1024, 32, True),    # ragged N, a full 32-row tile
+    (1000, 1024, 33, True),    # 64-row tiles, the first row of the second half
+    (257, 1152, 65, False),    # one column and one row past a tile, odd group count
+    (2560, 9728, 4, True),     # past the band kernel's LDS: the GEMM at 4 rows, split K
+    (2560, 9728, 200, True),   # split K over 64-row tiles
+])
+def test_int8_gemm(dev, stream, n, k, b, awq):
+    """The INT8 GEMM at the edges of its tiles, to test_int8_projection's bound."""
+    test_int8_projection(dev, stream, n, k, b, awq)
+
+
+def test_int8_capture_without_scratch(dev):
+    """A capture on a stream whose scratch cannot hold the GEMM's planes records the
+    scratch-free kernel: replays equal the eager GEMM within the bound, twice."""
+    n, k, b = 1000, 1024, 40
+    q, x = int8_problem(n, k, b, 77, True)
+    wt = ops.AffineInt8Weight(dev, q)
+    xd, ye, yg = dev.upload(x), dev.empty((b, n), np.float16), dev.empty((b, n), np.float16)
+    s = dev.stream()
+    g = s.capture(lambda: ops.encode_projection_int8(s, xd, wt, yg, b))
+    ops.encode_projection_int8(s, xd, wt, ye, b)
+    s.sync()
+    want = ye.read().astype(np.float64)
+    a = np.abs(x.astype(np.float64) / q.awq.astype(np.float64))
+    terms = a @ ((q.data + np.abs(q.zeros.astype(np.float64)).repeat(128, axis=1))
+                 * q.scales.astype(np.float64).repeat(128, axis=1)).T
+    for _ in range(2):
+        s.zero(yg)
+        g.launch()
+        s.sync()
+        # both sides are within a step + 2^-18 terms of the exact value
+        assert np.all(np.abs(yg.read().astype(np.float64) - want) <= 2 * (f16_step(want) + 2.0 ** -18 * terms))
+
+
 @pytest.mark.parametrize("t,k", [(1, 128), (1, 2560), (5, 9728), (64, 4096)])
 def test_quantize_input_q8_bit_exact(dev, stream, t, k):
     rng = np.random.default_rng(t * 7 + k)
