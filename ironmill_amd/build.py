@@ -19,7 +19,7 @@ OBJDIR = os.path.join(HERE, "_build")
 SOURCES = ["runtime.hip", "int4_matvec.hip", "int4_matvec_raw.hip", "int4_matvec_mt2.hip", "int4_matvec_band.hip", "int4_matvec_da.hip",
            "int4_gemm.hip",
            "int4_gemm_mx.hip", "int8_matvec.hip",
-           "tq_kernels.hip", "fp16_attention.hip", "glue_kernels.hip", "decoder.hip",
+           "tq_kernels.hip", "fp16_attention.hip", "prefill_attention.hip", "glue_kernels.hip", "decoder.hip",
            "tq_tables.cpp", "diag_probe.hip", "diag_valu_matvec.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -packed-fp32-ops: hipcc must not emit packed f32 VALU ops (they have given
@@ -40,6 +40,7 @@ FLAGS = [
 # (the softmax rescale touches them every chunk; AGPR copies would cost 64 VALU)
 EXTRA_FLAGS = {
     "tq_kernels.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "prefill_attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

@@ -25,6 +25,7 @@
 
 #include "dpp_reduce.h"
 #include "imh_internal.h"
+#include "prefill_attention.h"
 
 namespace {
 
@@ -307,6 +308,51 @@ int check_cache(const imh_fp16_kv_cache *c, const char *who) {
     return IMH_OK;
 }
 
+// token_count > 1: the row-tile kernel and, with several splits, the reduction.
+// A split that the scratch cannot hold while the stream captures is not made.
+int prefill_attention(imh_stream *stream, const imh_fp16_kv_cache *cache, const uint16_t *q, uint32_t num_heads,
+                      uint32_t gqa, uint32_t T, uint32_t seq_len, const int32_t *seq_lens, float attn_scale,
+                      uint16_t *out, uint32_t num_splits) {
+    const uint32_t nkv = cache->num_kv_heads, B = cache->batch;
+    const uint32_t L = seq_lens && seq_len == 0 ? cache->max_seq_len : seq_len;
+    const uint32_t rows = T * gqa;
+    const uint32_t tile = (uint32_t)imh::prefill_row_tile(false);
+    const uint32_t groups = B * nkv * ((rows + tile - 1) / tile);
+    uint32_t want = num_splits ? num_splits
+                               : imh::prefill_splits(false, groups, L, stream->dev->props.multiProcessorCount);
+    want = std::max<uint32_t>(1, std::min(want, (L + kSplitQuantum - 1) / kSplitQuantum));
+    uint32_t split_len = (L + want - 1) / want;
+    split_len = std::max<uint32_t>(kSplitQuantum, (split_len + kSplitQuantum - 1) / kSplitQuantum * kSplitQuantum);
+    uint32_t S = std::max<uint32_t>(1, (L + split_len - 1) / split_len);
+    const size_t nparts = (size_t)B * T * num_heads * S;
+    void *scr = nullptr;
+    if (S > 1 && !imh::stream_scratch_optional(stream, 1, nparts * (kD + 2) * sizeof(float), &scr)) {
+        S = 1;
+        split_len = std::max<uint32_t>(kSplitQuantum, (L + kSplitQuantum - 1) / kSplitQuantum * kSplitQuantum);
+    }
+    imh::PrefillAttention a = {};
+    a.q = reinterpret_cast<const _Float16 *>(q);
+    a.k = reinterpret_cast<const uint8_t *>(cache->k);
+    a.v = reinterpret_cast<const uint8_t *>(cache->v);
+    a.seq_lens = seq_lens;
+    a.part_o = static_cast<float *>(scr);
+    a.part_m = a.part_o + nparts * kD;
+    a.part_l = a.part_m + nparts;
+    a.out = reinterpret_cast<__half *>(out);
+    a.T = (int)T;
+    a.gqa = (int)gqa;
+    a.nh = (int)num_heads;
+    a.nkv = (int)nkv;
+    a.max_seq = (int)cache->max_seq_len;
+    a.seq_len = (int)L;
+    a.split_len = (int)split_len;
+    a.attn_scale = attn_scale;
+    const int rc = imh::launch_prefill_attention(stream, false, B, S, a);
+    if (rc || S == 1) return rc;
+    return imh::launch_prefill_combine(stream, false, (size_t)B * T * num_heads, S, a.part_o, a.part_m, a.part_l, nullptr,
+                                       a.out);
+}
+
 }  // namespace
 
 extern "C" {
@@ -359,6 +405,17 @@ int imh_encode_fp16_attention(imh_stream *stream, const imh_fp16_kv_cache *cache
         return imh::fail(IMH_EINVAL, std::string(who) + ": batch * token_count above 65535");
     rc = imh::use_device(stream->dev);
     if (rc) return rc;
+
+    // Several tokens: the row-tile kernel (a prefill chunk), except where the
+    // call has few query blocks (tokens of 4 rows, below) and this kernel, which
+    // gives each its own workgroups, is done sooner -- us, this : row tile, 8
+    // kv heads: 1 sequence at GQA 4, 16384 positions T = 2 29 : 48, 3 48 : 48,
+    // 5 64 : 49, 16 109 : 51; GQA 1, T = 16 (32 blocks) 40 : 49 but at 2048
+    // positions 19.6 : 18.6; 8 sequences at GQA 2, T = 2 103 : 102, 5 209 : 102
+    const uint32_t blocks = B * nkv * qblocks;
+    if (token_count > 1 && !(blocks <= 16 || (blocks <= 32 && seq_len >= 8192)))
+        return prefill_attention(stream, cache, q, num_heads, gqa, token_count, seq_len, seq_lens, attn_scale, out,
+                                 num_splits);
 
     // KV split: ~512 workgroups, each split a multiple of one pass of the
     // workgroup's waves (64 positions); with per-sequence lengths the splits

@@ -168,3 +168,26 @@ def test_attention_error_paths(dev, stream):
         ops.encode_fp16_kv_cache_and_attention(stream, cache, q, q, q, 32, 64, out)
     with pytest.raises(IronmillError, match="built for head_dim 128"):
         ops.encode_fp16_attention(stream, ops.Fp16KvCache(dev, 1, 8, 64, 64), q, 32, 1, out)
+
+
+@pytest.mark.parametrize("nh,nkv,tokens,num_splits,lens,shift", [
+    (32, 8, 33, 1, None, 0),          # 132 rows: four rows into a second row tile
+    (16, 8, 65, 0, (300, 40), 0),     # GQA 2; a sequence shorter than its tokens (rows without positions give 0)
+    (8, 8, 129, 2, (65, 300), 0),     # GQA 1; one position into a second position tile, an empty split
+    (32, 8, 40, 1, None, 2),          # q and out aligned to their elements only
+])
+def test_row_tile_kernel(dev, stream, nh, nkv, tokens, num_splits, lens, shift):
+    """The prefill kernel at the edges of its row and position tiles, against the oracle."""
+    batch, ctx, max_seq = 2, 300, 320
+    cache = fill_cache(dev, stream, batch, nkv, max_seq, ctx, seed=140 + tokens)
+    q16 = np.random.default_rng(tokens).standard_normal((batch, tokens, nh, D)).astype(np.float16)
+    qd, od = dev.buffer(q16.nbytes + 16), dev.buffer(q16.nbytes + 16)
+    qd.write(q16, shift)
+    sl = dev.upload(np.asarray(lens, np.int32)) if lens else None
+    ops.encode_fp16_attention(stream, cache, qd.ptr + shift, nh, ctx, od.ptr + shift, token_count=tokens,
+                              attn_scale=SCALE, seq_lens=sl, num_splits=num_splits)
+    stream.sync()
+    got = od.read(np.float16, q16.shape, shift)
+    ref = O.fp16_attention(q16, cache.k.read(), cache.v.read(), ctx, SCALE, nthreads=8,
+                           seq_lens=np.asarray(lens, np.int32) if lens else None)
+    assert_close(got, ref, what=f"row tiles T={tokens} nh={nh}")

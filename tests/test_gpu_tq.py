@@ -336,6 +336,32 @@ def test_attention_prefill_token_blocks(dev, stream, tq, tables, nh, tokens, num
         assert_close(got[:, t], ref, rel=5e-4, what=f"token {t} (lengths {lt.tolist()})")
 
 
+@pytest.mark.parametrize("num_splits", [0, 1, 3])
+def test_attention_prefill_row_tiles(dev, stream, tq, tables, num_splits):
+    """The row-tile prefill kernel (256 (token, head) rows per workgroup; chosen by the call's
+    size): tokens at the edges of its row tiles equal the one-token oracle at their own
+    lengths, for a full, a partial and a too short range; splits that hold nothing."""
+    nkv, nh, batch, max_seq, tokens = 8, 16, 4, 1024, 129
+    cache = fill_cache(dev, stream, tq, batch, nkv, max_seq, 900, seed=91)
+    q16 = np.random.default_rng(92).standard_normal((batch, tokens, nh, D)).astype(np.float16)
+    out = dev.empty((batch, tokens, nh, D), np.float16)
+    lens = np.array([900, 283, 100, 129], np.int32)
+    ops.encode_turboquant_attention(stream, tq, cache, dev.upload(q16), nh, 0, out, 1.0 / math.sqrt(D),
+                                    seq_lens=dev.upload(lens), num_splits=num_splits, token_count=tokens)
+    stream.sync()
+    got = out.read()
+    kc, vc, ks, vs, kr = read_cache(cache)
+    for t in (0, 1, 15, 16, 28, 29, 63, 64, 127, 128):
+        lt = np.maximum(lens - tokens + t + 1, 0).astype(np.int32)
+        ref = O.tq_attention(q16[:, t], tables, kc, vc, ks, vs, kr, max_seq, 1.0 / math.sqrt(D),
+                             seq_lens=lt, nthreads=8)
+        for bb in range(batch):
+            if lt[bb] == 0:
+                assert not got[bb, t].astype(np.float32).any()
+            else:
+                assert_close(got[bb, t], ref[bb], rel=5e-4, what=f"token {t} of seq {bb} (len {lt[bb]})")
+
+
 def test_graph_replay_after_scratch_growth(dev, tq):
     """A graph keeps addressing the stream scratch it was captured with: a larger eager op
     that grows the scratch afterwards must not free it (the replay equals the eager run,
