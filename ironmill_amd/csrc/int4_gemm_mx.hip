@@ -27,20 +27,28 @@
 //    so the fold of a group is one multiply-add.
 //  * a prep kernel writes the operand rows (x / awq rounded, each 8-element
 //    chunk in the slot order the code unpack produces) and their group sums.
+//    (INT4 codes beside a bf16 exponent: one and-or per two codes.)
 //  * the 32 x 32 matrix-core shapes (v_mfma_f32_32x32x16_bf16,
 //    v_mfma_scale_f32_32x32x64_f8f6f4): measured on the MI355X they sustain
 //    ~2.3 / ~4.9 PFLOP/s where the 16 x 16 bf16 shape stops at ~1.7.
-//  * workgroup tile 64 (M) x 256 columns, four waves each owning 64 x 64
-//    (2 x 2 MFMA tiles of 32 x 32); the next group's A (global -> registers
-//    -> other LDS buffer) and B (global -> registers) are loaded while the
-//    current group computes, their loads issued one or two per k step (a
-//    burst of twelve at the group's start held the wave's issue for ~400
-//    cycles), unconditionally (the last group re-loads itself), so no wait
-//    for them sits inside the compute: one barrier per group.  K is split over
-//    workgroups when the tile grid leaves workgroup slots (two per CU) idle
-//    and a model of the dispatch says the split pays for its partials; the
-//    f32 partials are summed in split order by a second kernel
+//  * the frame of wq_gemm.h, which says why: four waves of 64 rows x 64
+//    columns, A in LDS in operand order, double-buffered by group with one
+//    barrier per group; buffer resources with scalar group offsets and LDS
+//    immediates, so that the vector unit does little but expand codes and fold
+//    sums; loads held at their k step by scheduling barriers; scales and
+//    zero-points from a transposed copy that the prep launch writes.  The row
+//    sums' three pieces are formed once per group and row by the thread that
+//    stages them, not by every wave.
+//  * K is split over workgroups when the tile grid leaves workgroup slots (two
+//    per CU) idle and a model of the dispatch says the split pays for its
+//    partials; the f32 partials are summed in split order by a second kernel
 //    (deterministic).
+// Measured (us, AWQ, with the prep launch; before: row-major LDS rows, 64-bit
+// addresses and in-place scale reads): bf16 M = 2048 K 2560 -> N 9728 126 -> 122,
+// M = 1024 K 9728 -> N 2560 88 -> 79, M = 9 19.9 -> 16.9; fp8 M = 509 K 9728 ->
+// N 2560 49.5 -> 43.1, M = 1024 77.7 -> 64.3.  At M = 2048 what is left is the
+// matrix cores at their sustained clock (104 us with expansion and fold taken
+// out) and the 2.4 rounds of tiles.
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
@@ -49,21 +57,17 @@
 
 #include "dpp_reduce.h"
 #include "imh_internal.h"
+#include "wq_gemm.h"
 
 namespace {
 
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
-constexpr int kGS = 128;
-constexpr int kBM = 64;          // workgroup rows (M)
-constexpr int kThreads = 256;    // 4 waves, each owning 64 rows x 64 columns
-constexpr int kWaveCols = 64;    // two 32-column B fragments per wave
-template <int P> constexpr int wg_cols() { return 4 * kWaveCols; }
+using namespace imh_wq;
+
+constexpr int kCols = 256;       // columns per workgroup, 64 per wave
 constexpr float kE4M3Max = 448.0f;
 
 enum Prec : int { PREC_BF16 = 1, PREC_FP8 = 2 };
@@ -74,20 +78,53 @@ enum Prec : int { PREC_BF16 = 1, PREC_FP8 = 2 };
 constexpr uint32_t kScaleCodesE8m0 = 0x88888888u;
 constexpr uint32_t kScaleOneE8m0 = 0x7F7F7F7Fu;
 
-// grid (ceil(K / 8 / 256), M), block 256: chunk c (8 elements) of row m:
-// a = x / awq (no awq: x) rounded to the operand type, stored in slot order
-// {0, 2, 4, 6, 1, 3, 5, 7}; the 16 chunks of a group (16 consecutive lanes)
-// sum their rounded values into gsum[m][g].
+// the column constants of a group: scale f32, and the correction's factor -c
+// (c = 128 + z for the bf16 codes, which carry 128; z for fp8) as a bf16 pair
+template <int P>
+__device__ __forceinline__ u32x2_t mx_consts(uint16_t s, uint16_t z) {
+    const __bf16 c = (__bf16)((P == PREC_BF16 ? -128.0f : 0.0f) - (float)__builtin_bit_cast(_Float16, z));
+    const uint32_t cb = __builtin_bit_cast(uint16_t, c);
+    return (u32x2_t){__builtin_bit_cast(uint32_t, (float)__builtin_bit_cast(_Float16, s)), cb | (cb << 16)};
+}
+
+// Workgroups below ablocks: chunk c (8 elements) of the rows: a = x / awq (no
+// awq: x) rounded to the operand type, stored in the order the code expansion
+// yields (bf16 {0, 4, 1, 5, 2, 6, 3, 7}, fp8 {0, 2, 4, 6, 1, 3, 5, 7}); the 16
+// chunks of a group (16 consecutive lanes) sum their rounded values into
+// gsum[m][g].  The others transpose 64 columns x 16 groups of the scales and
+// zero-points into szt[group][column].
 template <int P>
 __global__ void __launch_bounds__(256) gemm_mx_prep_kernel(const __bf16 *__restrict__ x,
                                                            const __half *__restrict__ awq,
                                                            uint8_t *__restrict__ aop, float *__restrict__ gsum,
-                                                           int K) {
-    const int m = blockIdx.y;
-    const int c_raw = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = c_raw * 8 < K;
-    const int c = live ? c_raw : 0;
-    const size_t off = (size_t)m * K + (size_t)c * 8;
+                                                           size_t chunks, int K, int ablocks,
+                                                           const uint16_t *__restrict__ scales,
+                                                           const uint16_t *__restrict__ zeros,
+                                                           u32x2_t *__restrict__ szt, int N) {
+    if ((int)blockIdx.x >= ablocks) {
+        const int G = K / kGS, gblk = (G + 15) / 16, blk = (int)blockIdx.x - ablocks;
+        const int n = (blk / gblk) * 64 + (int)(threadIdx.x & 63);
+        const int g0 = (blk % gblk) * 16 + (int)(threadIdx.x >> 6) * 4;
+        if (n >= N) return;
+        uint16_t sv[4], zv[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const size_t at = (size_t)n * G + min(g0 + i, G - 1);
+            sv[i] = scales[at];
+            zv[i] = zeros[at];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (g0 + i < G) szt[(size_t)(g0 + i) * N + n] = mx_consts<P>(sv[i], zv[i]);
+        return;
+    }
+    const size_t cr = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const bool live = cr < chunks;
+    const size_t ca = live ? cr : 0;
+    const int cpr = K / 8;
+    const size_t m = ca / cpr;
+    const int c = (int)(ca - m * cpr);
+    const size_t off = ca * 8;
     const u32x4_t xv = *reinterpret_cast<const u32x4_t *>(x + off);
     const __bf16 *xb = reinterpret_cast<const __bf16 *>(&xv);
     float v[8];
@@ -99,13 +136,13 @@ __global__ void __launch_bounds__(256) gemm_mx_prep_kernel(const __bf16 *__restr
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] = v[i] / (float)wh[i];
     }
-    constexpr int kSlot[8] = {0, 2, 4, 6, 1, 3, 5, 7};
+    constexpr int kSlot4[8] = {0, 4, 1, 5, 2, 6, 3, 7}, kSlot8[8] = {0, 2, 4, 6, 1, 3, 5, 7};
     float sum = 0.0f;
     if (P == PREC_BF16) {
         bf16x8_t o;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            o[i] = (__bf16)v[kSlot[i]];
+            o[i] = (__bf16)v[kSlot4[i]];
             sum += (float)o[i];
         }
         if (live) *reinterpret_cast<bf16x8_t *>(aop + off * 2) = o;
@@ -115,7 +152,7 @@ __global__ void __launch_bounds__(256) gemm_mx_prep_kernel(const __bf16 *__restr
         for (int h = 0; h < 2; h++) {
             float e[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) e[i] = fminf(fmaxf(v[kSlot[4 * h + i]], -kE4M3Max), kE4M3Max);
+            for (int i = 0; i < 4; i++) e[i] = fminf(fmaxf(v[kSlot8[4 * h + i]], -kE4M3Max), kE4M3Max);
             uint32_t p = __builtin_amdgcn_cvt_pk_fp8_f32(e[0], e[1], 0, false);
             p = __builtin_amdgcn_cvt_pk_fp8_f32(e[2], e[3], p, true);
             w[h] = p;
@@ -133,29 +170,6 @@ __global__ void __launch_bounds__(256) gemm_mx_prep_kernel(const __bf16 *__restr
     if (live && (threadIdx.x & 15) == 0) gsum[(size_t)m * (K / kGS) + (size_t)c / 16] = sum;
 }
 
-// Tile order.  Workgroup ids go round-robin over the 8 XCDs, each with its
-// own L2, so the linear id is first turned into an index that is contiguous
-// per XCD; that index then walks bands of `band` row tiles (M) with the row
-// tile fastest, so the workgroups resident on one XCD share both their A rows
-// (one band) and their B columns (neighbouring column tiles) in its L2.
-struct TileOrder {
-    int tiles_m, tiles_n, band, splits;
-};
-__device__ __forceinline__ void tile_of(const TileOrder &o, int &mt, int &nt, int &split) {
-    const int T = o.tiles_m * o.tiles_n * o.splits;
-    const int L = blockIdx.x;
-    const int x = L & 7, j = L >> 3;
-    const int q = T >> 3, r = T & 7;
-    const int t = x * q + min(x, r) + j;             // contiguous per XCD
-    const int per_split = o.tiles_m * o.tiles_n;
-    split = t / per_split;
-    const int u = t - split * per_split;
-    const int per_band = o.band * o.tiles_n;
-    const int b = u / per_band, v = u - b * per_band;
-    mt = b * o.band + v % o.band;
-    nt = v / o.band;
-}
-
 // grid (tiles_m * tiles_n * splits), block 256; tile (mt, nt, split) from
 // tile_of.  Split z covers groups [z * per, min((z + 1) * per, G)).  Without a
 // split C is stored as bf16; with one the f32 partials go to part[z][M][N].
@@ -164,24 +178,26 @@ __device__ __forceinline__ void tile_of(const TileOrder &o, int &mt, int &nt, in
 //   bf16 32x32x16, k step s (0..7) of a group: lane (n, h) holds the 8 codes
 //     [64 h + 8 s, +8) of column n -- dword s of the 32 code bytes
 //     [32 h, 32 h + 32) of the group row -- and A lane (m, h) the operand
-//     chunk 8 h + s of row m (8 elements in the code unpack's slot order);
+//     chunk 8 h + s of row m;
 //   fp8 32x32x64, k step t (0..1): lane (n, h) the 32 codes [64 t + 32 h, +32)
 //     (code bytes [32 t + 16 h, +16)), A lane (m, h) the 32 operand bytes at
-//     64 t + 32 h of row m;
+//     64 t + 32 h of row m (chunks 4 t + 2 h, + 1);
 //   D: lane l, value i: row 8 (i >> 2) + 4 h + (i & 3), column l & 31.
-template <int P>
+// LDS: block (row / 32, k step) of 64 lanes x 16 bytes -- fp8: (row / 32, k
+// step, half of the 32 bytes) -- padded by 16 bytes.
+template <int P, int MI, bool SZT>
 __global__ void __launch_bounds__(kThreads, 2) gemm_mx_kernel(
     const uint8_t *__restrict__ aop, const float *__restrict__ gsum, const uint8_t *__restrict__ wdata,
-    const __half *__restrict__ scales, const __half *__restrict__ zeros, __bf16 *__restrict__ out,
-    float *__restrict__ part, int M, int N, int K, int per, TileOrder order) {
+    const uint16_t *__restrict__ scales, const uint16_t *__restrict__ zeros, const u32x2_t *__restrict__ szt,
+    __bf16 *__restrict__ out, float *__restrict__ part, int M, int N, int K, int per, TileOrder order) {
+    constexpr int BM = 32 * MI;
     constexpr int EB = P == PREC_BF16 ? 2 : 1;     // operand bytes per element
-    constexpr int RB = kGS * EB + 16;              // LDS row bytes of one group (16-byte pad)
-    constexpr int ACH = kBM * kGS * EB / 16 / kThreads;   // 16-byte A chunks per thread per group
-    // A stages: [stage buffer][group of the stage] -- GPB groups per barrier:
-    // two at bf16, four at fp8 (its operand is half the bytes: the same LDS)
-    constexpr int GPB = P == PREC_BF16 ? 2 : 4;
-    __shared__ __attribute__((aligned(16))) uint8_t As[2][GPB][kBM * RB];
-    __shared__ __attribute__((aligned(16))) float Gs[2][GPB][kBM];
+    constexpr int CPR = kGS * EB / 16;             // 16-byte chunks of a row's group
+    constexpr int NBLK = CPR / 2;                  // LDS blocks per 32 rows
+    constexpr int RPP = kThreads / CPR;            // rows staged per pass
+    constexpr int ACH = BM / RPP;                  // chunks per thread and group
+    __shared__ __attribute__((aligned(16))) uint8_t As[2][MI * NBLK * kBlk];
+    __shared__ __attribute__((aligned(16))) u32x4_t Cs[2][BM];   // row sums in three bf16 pieces
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -189,244 +205,258 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_mx_kernel(
     const int nl = lane & 31, h = lane >> 5;
     int mt, nt, split;
     tile_of(order, mt, nt, split);
-    const int m0 = mt * kBM;
-    const int n0 = nt * wg_cols<P>() + wave * kWaveCols;
+    const int m0 = mt * BM;
+    const int nb = nt * kCols;
+    const int n0 = nb + wave * 64;
     const int G = K / kGS;
     const int g_begin = split * per;
     const int g_end = min(g_begin + per, G);
 
-    // B rows of this lane: fragment j holds column n0 + 32 j + nl (clamped)
-    const uint8_t *brow[2];
-    size_t szrow[2];
+    const int row_bytes = K / 2;
+    const int cols = min(kCols, N - nb);
+    const __amdgpu_buffer_rsrc_t w_r = __builtin_amdgcn_make_buffer_rsrc((void *)(wdata + (size_t)nb * row_bytes), 0,
+                                                                         cols * row_bytes, kRsrcWord3);
+    __amdgpu_buffer_rsrc_t s_r, z_r;
+    if (SZT) {
+        s_r = z_r = __builtin_amdgcn_make_buffer_rsrc((void *)(szt + nb), 0,
+                                                      (int)(((size_t)G * N - nb) * sizeof(u32x2_t)), kRsrcWord3);
+    } else {
+        s_r = __builtin_amdgcn_make_buffer_rsrc((void *)(scales + (size_t)nb * G), 0, cols * G * 2, kRsrcWord3);
+        z_r = __builtin_amdgcn_make_buffer_rsrc((void *)(zeros + (size_t)nb * G), 0, cols * G * 2, kRsrcWord3);
+    }
+    int bvo[2], svo[2];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-        const int n = min(n0 + 32 * j + nl, N - 1);
-        brow[j] = wdata + (size_t)n * (K / 2) + (P == PREC_BF16 ? 32 * h : 16 * h);
-        szrow[j] = (size_t)n * G;
+        const int n = min(n0 + 32 * j + nl, N - 1) - nb;
+        bvo[j] = n * row_bytes + (P == PREC_BF16 ? 32 : 16) * h;
+        svo[j] = SZT ? n * (int)sizeof(u32x2_t) : n * G * 2;
     }
-    // A staging: chunk c = i * 256 + tid of the group's 64 x (128 * EB) bytes
-    auto load_a1 = [&](int g, int i, u32x4_t *ar) __attribute__((always_inline)) {
-        const int c = i * kThreads + tid;
-        const int r = c / (kGS * EB / 16), cc = c - r * (kGS * EB / 16);
-        const int m = min(m0 + r, M - 1);
-        ar[i] = *reinterpret_cast<const u32x4_t *>(aop + ((size_t)m * K + (size_t)g * kGS) * EB + cc * 16);
-    };
-    auto load_gs = [&](int g, float &gs) __attribute__((always_inline)) {
-        gs = tid < kBM ? gsum[(size_t)min(m0 + tid, M - 1) * G + g] : 0.0f;
-    };
-    auto load_a = [&](int g, u32x4_t *ar, float &gs) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < ACH; i++) load_a1(g, i, ar);
-        load_gs(g, gs);
-    };
-    auto store_a = [&](int sb, int part, const u32x4_t *ar, float gs) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < ACH; i++) {
-            const int c = i * kThreads + tid;
-            const int r = c / (kGS * EB / 16), cc = c - r * (kGS * EB / 16);
-            *reinterpret_cast<u32x4_t *>(&As[sb][part][r * RB + cc * 16]) = ar[i];
-        }
-        if (tid < kBM) Gs[sb][part][tid] = gs;
-    };
-    // B codes (32 bytes per fragment and lane), scales and zero-points of
-    // group g; the scale and zero stay apart until used
     struct BRegs {
         u32x4_t w[2][2];
-        uint16_t s[2], z[2];
-    };
-    auto load_b1 = [&](int g, int j, BRegs &b) __attribute__((always_inline)) {
-        {
-            const uint8_t *p = brow[j] + (size_t)g * 64;
-            b.w[j][0] = *reinterpret_cast<const u32x4_t *>(p);
-            b.w[j][1] = *reinterpret_cast<const u32x4_t *>(p + (P == PREC_BF16 ? 16 : 32));
-            b.s[j] = reinterpret_cast<const uint16_t *>(scales)[szrow[j] + g];
-            b.z[j] = reinterpret_cast<const uint16_t *>(zeros)[szrow[j] + g];
-        }
     };
     auto load_b = [&](int g, BRegs &b) __attribute__((always_inline)) {
-        load_b1(g, 0, b);
-        load_b1(g, 1, b);
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                b.w[j][i] = __builtin_bit_cast(
+                    u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(w_r, bvo[j] + i * (P == PREC_BF16 ? 16 : 32), g * 64, 0));
+    };
+    auto load_c = [&](int g, u32x2_t *c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            if (SZT) {
+                c[j] = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(
+                                                       s_r, svo[j], g * N * (int)sizeof(u32x2_t), 0));
+            } else {
+                c[j][0] = __builtin_amdgcn_raw_buffer_load_b16(s_r, svo[j], g * 2, 0);
+                c[j][1] = __builtin_amdgcn_raw_buffer_load_b16(z_r, svo[j], g * 2, 0);
+            }
+        }
+    };
+    // A: pass i of a thread is row RPP i + tid / CPR, chunk tid % CPR; rows past M read as zeros
+    const int arows = min(BM, M - m0);
+    const __amdgpu_buffer_rsrc_t a_r = __builtin_amdgcn_make_buffer_rsrc((void *)(aop + (size_t)m0 * K * EB), 0,
+                                                                         arows * K * EB, kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t r_r =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(gsum + (size_t)m0 * G), 0, arows * G * 4, kRsrcWord3);
+    const int ar0 = tid / CPR, ac = tid % CPR;
+    const int avo = ar0 * K * EB + ac * 16;
+    const int ablk = P == PREC_BF16 ? (ac & 7) : 2 * (ac >> 2) + (ac & 1);
+    const int ah = P == PREC_BF16 ? ac >> 3 : (ac >> 1) & 1;
+    const int a_lds = ablk * kBlk + (ar0 + 32 * ah) * 16;
+    const int rvo = (tid & (BM - 1)) * G * 4;
+    auto load_a = [&](int g, u32x4_t *ar, float &rs) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < ACH; i++)
+            ar[i] = __builtin_bit_cast(
+                u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(a_r, avo, (g * kGS + i * RPP * K) * EB, 0));
+        rs = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_r, rvo, g * 4, 0));
+    };
+    auto store_a = [&](int buf, const u32x4_t *ar, float rs) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < ACH; i++) {
+            const int r = RPP * i;   // of the thread's rows, the part that is the same for all
+            *reinterpret_cast<u32x4_t *>(&As[buf][a_lds + (r >> 5) * NBLK * kBlk + (r & 31) * 16]) = ar[i];
+        }
+        // rs = r0 + r1 + r2 exactly, in bf16 (the same value from each wave)
+        const __bf16 r0 = (__bf16)rs;
+        const float e1 = rs - (float)r0;
+        const __bf16 r1 = (__bf16)e1;
+        const __bf16 r2 = (__bf16)(e1 - (float)r1);
+        Cs[buf][tid & (BM - 1)] =
+            (u32x4_t){(uint32_t)__builtin_bit_cast(uint16_t, r0) | ((uint32_t)__builtin_bit_cast(uint16_t, r1) << 16),
+                      (uint32_t)__builtin_bit_cast(uint16_t, r2), 0u, 0u};
     };
 
-    float16_t acc[2][2];
+    float16_t acc[MI][2];
 #pragma unroll
-    for (int mi = 0; mi < 2; mi++)
+    for (int mi = 0; mi < MI; mi++)
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[mi][j][i] = 0.0f;
 
-    // One group: the MFMAs of the four 32 x 32 tiles over the group's k
-    // steps, then each tile's group partial folded into acc with the scale
-    // and zero-point of the lane's column and the group sums of its rows.
-    // hook(st) runs at k step st: it issues the next group's loads.
-    auto compute = [&](int sb, int part, const BRegs &b, auto &&hook) __attribute__((always_inline)) {
-        const uint8_t *Ab = As[sb][part];
-        // The group's zero-point correction -c * rowsum (c = 128 + z for the
-        // bf16 codes, which carry 128; z for fp8) is added to each tile's
-        // group accumulator on the matrix core: A lane (m, 0) holds the row sum
-        // split into three bf16 pieces (hi + mid + lo == rowsum exactly), B
-        // lane (n, 0) -c three times (exact in bf16), all other k slots zero
-        // -- so the fold is one multiply-add per output.
-        bf16x8_t ca[2], cb[2];
-        {
-            const __bf16 z0 = (__bf16)0.0f;
+    // in registers, so that each and-or is one instruction
+    uint32_t m_lo, exp128;
+    asm("s_mov_b32 %0, 0x000f000f" : "=s"(m_lo));
+    asm("v_mov_b32 %0, 0x43004300" : "=v"(exp128));
+
+    // One group from LDS buffer buf: the MFMAs of the tiles over the group's k
+    // steps (hook(st): the next group's loads at k step st), the zero-point
+    // correction -c * rowsum as one more product (A lane (m, h): the row sum's
+    // three pieces, B lane (n, 0): -c three times, exact in bf16, lane (n, 1):
+    // zeros), then the fold with the scale of the lane's column.
+    auto compute = [&](int buf, const BRegs &b, const u32x2_t *cc, auto &&hook) __attribute__((always_inline)) {
+        float sc[2];
+        bf16x8_t cb[2];
 #pragma unroll
-            for (int mi = 0; mi < 2; mi++) {
-                const float rs = Gs[sb][part][32 * mi + nl];
-                const __bf16 r0 = (__bf16)rs;
-                const float e1 = rs - (float)r0;
-                const __bf16 r1 = (__bf16)e1;
-                const __bf16 r2 = (__bf16)(e1 - (float)r1);
-                ca[mi] = h == 0 ? (bf16x8_t){r0, r1, r2, z0, z0, z0, z0, z0} : (bf16x8_t){z0, z0, z0, z0, z0, z0, z0, z0};
-            }
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const __bf16 c = (__bf16)((P == PREC_BF16 ? -128.0f : 0.0f) - (float)__builtin_bit_cast(_Float16, b.z[j]));
-                cb[j] = h == 0 ? (bf16x8_t){c, c, c, z0, z0, z0, z0, z0} : (bf16x8_t){z0, z0, z0, z0, z0, z0, z0, z0};
-            }
+        for (int j = 0; j < 2; j++) {
+            const u32x2_t c = SZT ? cc[j] : mx_consts<P>((uint16_t)cc[j][0], (uint16_t)cc[j][1]);
+            const uint32_t cs = c[0], cz = h ? 0u : c[1];   // scalars: a bit cast of a vector element takes element 0
+            sc[j] = __builtin_bit_cast(float, cs);
+            cb[j] = __builtin_bit_cast(bf16x8_t, (u32x4_t){cz, cz & 0xFFFFu, 0u, 0u});
         }
+        const uint8_t *ab = &As[buf][lane * 16];
+        bf16x8_t ca[MI];
+        auto read_c = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++) ca[mi] = __builtin_bit_cast(bf16x8_t, Cs[buf][32 * mi + nl]);
+        };
         const float16_t zero16 = {};
-        if (P == PREC_BF16) {
-            float16_t gg[2][2];
+        if constexpr (P == PREC_BF16) {
+            bf16x8_t af[2][MI], bf[2][2];
+            auto read_a = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
-            for (int st = 0; st < 8; st++) {
-                hook(st);
-                bf16x8_t af[2], bf[2];
-#pragma unroll
-                for (int mi = 0; mi < 2; mi++)
-                    af[mi] = *reinterpret_cast<const bf16x8_t *>(&Ab[(32 * mi + nl) * RB + (8 * h + st) * 16]);
+                for (int mi = 0; mi < MI; mi++)
+                    af[st & 1][mi] = *reinterpret_cast<const bf16x8_t *>(ab + (mi * NBLK + st) * kBlk);
+            };
+            // 8 codes -> bf16 128 + q in slot order {0, 4, 1, 5, 2, 6, 3, 7}
+            auto expand = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
-                    // 8 codes -> bf16 128 + q in slot order {0, 2, 4, 6, 1, 3, 5, 7}
                     const uint32_t w = b.w[j][st >> 2][st & 3];
-                    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-                    const u32x4_t o = {__builtin_amdgcn_perm(lo, 0x43434343u, 0x00050004u),
-                                       __builtin_amdgcn_perm(lo, 0x43434343u, 0x00070006u),
-                                       __builtin_amdgcn_perm(hi, 0x43434343u, 0x00050004u),
-                                       __builtin_amdgcn_perm(hi, 0x43434343u, 0x00070006u)};
-                    bf[j] = __builtin_bit_cast(bf16x8_t, o);
+                    bf[st & 1][j] = __builtin_bit_cast(
+                        bf16x8_t, (u32x4_t){(w & m_lo) | exp128, ((w >> 4) & m_lo) | exp128, ((w >> 8) & m_lo) | exp128,
+                                            ((w >> 12) & m_lo) | exp128});
                 }
+            };
+            float16_t gg[MI][2];
+            read_a(0);
+            expand(0);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int mi = 0; mi < 2; mi++)
+            for (int st = 0; st < 8; st++) {
+                if (st < 7) read_a(st + 1);
+                else read_c();
+                hook(st);
+                if (st < 7) expand(st + 1);
+#pragma unroll
+                for (int mi = 0; mi < MI; mi++)
 #pragma unroll
                     for (int j = 0; j < 2; j++)
-                        gg[mi][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[mi], bf[j], st == 0 ? zero16 : gg[mi][j],
-                                                                            0, 0, 0);
+                        gg[mi][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[st & 1][mi], bf[st & 1][j],
+                                                                            st == 0 ? zero16 : gg[mi][j], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            // the zero-point correction last: its operands (an LDS read and a
-            // short VALU chain) are built while the k steps run, not ahead of them
 #pragma unroll
-            for (int mi = 0; mi < 2; mi++)
+            for (int mi = 0; mi < MI; mi++)
 #pragma unroll
                 for (int j = 0; j < 2; j++)
                     gg[mi][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca[mi], cb[j], gg[mi][j], 0, 0, 0);
 #pragma unroll
-            for (int mi = 0; mi < 2; mi++)
+            for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const float sj = (float)__builtin_bit_cast(_Float16, b.s[j]);
+                for (int j = 0; j < 2; j++)
 #pragma unroll
-                    for (int i = 0; i < 16; i++) acc[mi][j][i] = __builtin_fmaf(sj, gg[mi][j][i], acc[mi][j][i]);
-                }
+                    for (int i = 0; i < 16; i++) acc[mi][j][i] = __builtin_fmaf(sc[j], gg[mi][j][i], acc[mi][j][i]);
         } else {
+            i32x8_t af[2][MI], bf[2][2];
+            auto read_a = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-            for (int st = 0; st < 6; st++) hook(st);
-            // both k steps' A fragments, then per column fragment its B
-            // fragments and the two tiles' MFMAs: one tile's partial live at a time
-            i32x8_t af[2][2];
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int mi = 0; mi < 2; mi++) {
-                    const uint8_t *p = &Ab[(32 * mi + nl) * RB + 64 * t + 32 * h];
-                    const u32x4_t a0 = *reinterpret_cast<const u32x4_t *>(p);
-                    const u32x4_t a1 = *reinterpret_cast<const u32x4_t *>(p + 16);
-                    af[mi][t] = (i32x8_t){(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3],
+                for (int mi = 0; mi < MI; mi++) {
+                    const u32x4_t a0 = *reinterpret_cast<const u32x4_t *>(ab + (mi * NBLK + 2 * t) * kBlk);
+                    const u32x4_t a1 = *reinterpret_cast<const u32x4_t *>(ab + (mi * NBLK + 2 * t + 1) * kBlk);
+                    af[t][mi] = (i32x8_t){(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3],
                                           (int)a1[0], (int)a1[1], (int)a1[2], (int)a1[3]};
                 }
+            };
+            // code dword d = codes 8 d .. 8 d + 7 -> the even codes' bytes, then the odd
+            auto expand = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                i32x8_t bf[2];
-#pragma unroll
-                for (int t = 0; t < 2; t++)
-                    // code dword d = codes 8 d .. 8 d + 7 -> the even codes' bytes, then the odd
+                for (int j = 0; j < 2; j++)
 #pragma unroll
                     for (int d = 0; d < 4; d++) {
                         const uint32_t w = b.w[j][t][d];
-                        bf[t][2 * d] = (int)(w & 0x0F0F0F0Fu);
-                        bf[t][2 * d + 1] = (int)((w >> 4) & 0x0F0F0F0Fu);
+                        bf[t][j][2 * d] = (int)(w & 0x0F0F0F0Fu);
+                        bf[t][j][2 * d + 1] = (int)((w >> 4) & 0x0F0F0F0Fu);
                     }
-                const float sj = (float)__builtin_bit_cast(_Float16, b.s[j]);
+            };
+            float16_t gg[MI][2];
+            read_c();
+            read_a(0);
+            expand(0);
+            __builtin_amdgcn_sched_barrier(0);
+            hook(0);
 #pragma unroll
-                for (int mi = 0; mi < 2; mi++) {
-                    float16_t g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca[mi], cb[j], zero16, 0, 0, 0);
+            for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-                    for (int t = 0; t < 2; t++)
-                        // formats 0 / 0: e4m3 x e4m3; A scale x1, B scale x 2^9
-                        g = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af[mi][t], bf[t], g, 0, 0, 0, kScaleOneE8m0,
-                                                                            0, kScaleCodesE8m0);
+                for (int j = 0; j < 2; j++)
+                    gg[mi][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca[mi], cb[j], zero16, 0, 0, 0);
+            read_a(1);
+            expand(1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int i = 0; i < 16; i++) acc[mi][j][i] = __builtin_fmaf(sj, g[i], acc[mi][j][i]);
-                }
+            for (int t = 0; t < 2; t++) {
+                hook(t + 1);
+                // formats 0 / 0: e4m3 x e4m3; A scale x1, B scale x 2^9
+#pragma unroll
+                for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        gg[mi][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                            af[t][mi], bf[t][j], gg[mi][j], 0, 0, 0, kScaleOneE8m0, 0, kScaleCodesE8m0);
+                __builtin_amdgcn_sched_barrier(0);
             }
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[mi][j][i] = __builtin_fmaf(sc[j], gg[mi][j][i], acc[mi][j][i]);
         }
     };
 
-    // Ping-pong over two B register sets (no copies between iterations), A in
-    // stages of two groups with one barrier per stage: group g computes from
-    // stage buffer sb (part g & 1 of the stage) while group g + 2's A is
-    // loaded into registers and, after g's MFMAs, stored to the other stage
-    // buffer -- free since the barrier that closed the stage before (every
-    // wave was done reading it) -- and group g + 1's B into the other set.
-    // The prefetch is unconditional -- past the last group the last one is
-    // loaded again -- so the compiler's wait for the current set never has to
-    // cover the prefetch.
     u32x4_t ar[ACH];
+    float rs = 0.0f;
     BRegs b0, b1;
-    float gsv = 0.0f;
+    u32x2_t c0[2], c1[2];
     if (g_begin < g_end) {
-        load_a(g_begin, ar, gsv);
         load_b(g_begin, b0);
-        store_a(0, 0, ar, gsv);
-#pragma unroll
-        for (int q = 1; q < GPB; q++) {
-            load_a(min(g_begin + q, g_end - 1), ar, gsv);
-            store_a(0, q, ar, gsv);
-        }
+        load_c(g_begin, c0);
+        load_a(g_begin, ar, rs);
+        store_a(0, ar, rs);
         __syncthreads();
     }
-    auto step = [&](int g, int sb, int part, const BRegs &cur, BRegs &nxt) __attribute__((always_inline)) {
-        const int ga = min(g + GPB, g_end - 1), gb = min(g + 1, g_end - 1);
-        // the loads spread over the k steps: A chunks first (they are stored
-        // to LDS after the compute), then B
-        compute(sb, part, cur, [&](int st) __attribute__((always_inline)) {
-            if (st < ACH) load_a1(ga, st, ar);
-            if (st == ACH) load_gs(ga, gsv);
-            if (st == 4) load_b1(gb, 0, nxt);
-            if (st == 5) load_b1(gb, 1, nxt);
-        });
-        store_a(sb ^ 1, part, ar, gsv);
-    };
-    // two stages per iteration: the stage buffers' indices are constants (GPB
-    // is even, so group parity and part parity pick the same B set)
-    for (int g = g_begin; g < g_end; g += 2 * GPB) {
-#pragma unroll
-        for (int q = 0; q < GPB; q++) {
-            if (g + q >= g_end) break;
-            if (q & 1) step(g + q, 0, q, b1, b0);
-            else step(g + q, 0, q, b0, b1);
-        }
-        __syncthreads();
-        if (g + GPB < g_end) {
-#pragma unroll
-            for (int q = 0; q < GPB; q++) {
-                if (g + GPB + q >= g_end) break;
-                if (q & 1) step(g + GPB + q, 1, q, b1, b0);
-                else step(g + GPB + q, 1, q, b0, b1);
+    // the next group's loads are unconditional (past the last group the last
+    // one is loaded again), so no wait for the current set has to cover them
+    auto step = [&](int g, int buf, const BRegs &cur, const u32x2_t *cc, BRegs &nxt,
+                    u32x2_t *nc) __attribute__((always_inline)) {
+        const int gn = min(g + 1, g_end - 1);
+        compute(buf, cur, cc, [&](int st) __attribute__((always_inline)) {
+            if (st == 0) load_a(gn, ar, rs);
+            if (st == 1) {
+                load_b(gn, nxt);
+                load_c(gn, nc);
             }
-            __syncthreads();
-        }
+        });
+        store_a(buf ^ 1, ar, rs);
+        __syncthreads();
+    };
+    for (int g = g_begin; g < g_end; g += 2) {
+        step(g, 0, b0, c0, b1, c1);
+        if (g + 1 >= g_end) break;
+        step(g + 1, 1, b1, c1, b0, c0);
     }
 
     // D of tile (mi, j): lane holds rows 32 mi + 8 (i >> 2) + 4 h + (i & 3), column 32 j + nl
@@ -435,7 +465,7 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_mx_kernel(
         const int n = n0 + 32 * j + nl;
         if (n >= N) continue;
 #pragma unroll
-        for (int mi = 0; mi < 2; mi++)
+        for (int mi = 0; mi < MI; mi++)
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int m = m0 + 32 * mi + 8 * (i >> 2) + 4 * h + (i & 3);
@@ -529,38 +559,15 @@ int imh_affine_gemm_int4(imh_stream *stream, const void *x, uint32_t M, const im
     const int N = (int)w->n, K = (int)w->k, G = K / kGS;
     const int P = precision == IMH_GEMM_BF16 ? PREC_BF16 : PREC_FP8;
     const int eb = P == PREC_BF16 ? 2 : 1;
-    // K split (fewer tiles than workgroup slots, two per CU)
     const int cus = stream->dev->props.multiProcessorCount;
-    const int wgc = P == PREC_BF16 ? wg_cols<PREC_BF16>() : wg_cols<PREC_FP8>();
-    const int tiles = ((N + wgc - 1) / wgc) * (((int)M + kBM - 1) / kBM);
+    const int bm = M <= 32 ? 32 : 64;
+    TileOrder order;
+    order.tiles_m = ((int)M + bm - 1) / bm;
+    order.tiles_n = (N + kCols - 1) / kCols;
+    const int tiles = order.tiles_m * order.tiles_n;
     int splits = tiles < 2 * cus ? gemm_splits(tiles, G, (int)M, N, cus, P) : 1;
     const int per = (G + splits - 1) / splits;
     splits = (G + per - 1) / per;
-    // scratch slot 0: operand rows + group sums; slot 2: split partials
-    const size_t a_bytes = ((size_t)M * K * eb + 255) / 256 * 256;
-    void *scr = nullptr;
-    rc = imh::stream_scratch(stream, 0, a_bytes + (size_t)M * G * sizeof(float), &scr);
-    if (rc) return rc;
-    uint8_t *aop = static_cast<uint8_t *>(scr);
-    float *gsum = reinterpret_cast<float *>(aop + a_bytes);
-    float *part = nullptr;
-    if (splits > 1) {
-        void *p = nullptr;
-        rc = imh::stream_scratch(stream, 2, (size_t)splits * M * N * sizeof(float), &p);
-        if (rc) return rc;
-        part = static_cast<float *>(p);
-    }
-    const __bf16 *xb = static_cast<const __bf16 *>(x);
-    const __half *awq = reinterpret_cast<const __half *>(w->awq_scales);
-    dim3 pgrid((K / 8 + 255) / 256, M);
-    if (P == PREC_BF16)
-        hipLaunchKernelGGL(gemm_mx_prep_kernel<PREC_BF16>, pgrid, dim3(256), 0, stream->stream, xb, awq, aop, gsum, K);
-    else
-        hipLaunchKernelGGL(gemm_mx_prep_kernel<PREC_FP8>, pgrid, dim3(256), 0, stream->stream, xb, awq, aop, gsum, K);
-    IMH_HIP(hipGetLastError());
-    TileOrder order;
-    order.tiles_m = ((int)M + kBM - 1) / kBM;
-    order.tiles_n = (N + wgc - 1) / wgc;
     order.splits = splits;
     // band: the largest divisor of tiles_m that is at most tiles_m / 8 (so
     // each XCD gets about one band), at least 1
@@ -570,15 +577,57 @@ int imh_affine_gemm_int4(imh_stream *stream, const void *x, uint32_t M, const im
             order.band = b;
             break;
         }
-    dim3 grid((unsigned)order.tiles_m * order.tiles_n * splits);
-    const __half *sc = reinterpret_cast<const __half *>(w->scales), *zr = reinterpret_cast<const __half *>(w->zeros);
+    // scratch slot 0: operand rows, group sums and, where it has room, the
+    // transposed column constants (a stream capturing with the scratch of the
+    // first two reads scales and zero-points in place); slot 2: split partials
+    const size_t a_bytes = ((size_t)M * K * eb + 255) / 256 * 256;
+    const size_t gsum_bytes = ((size_t)M * G * sizeof(float) + 255) / 256 * 256;
+    const size_t szt_bytes = (size_t)G * N * sizeof(u32x2_t);
+    void *scr = nullptr;
+    const bool has_szt = szt_bytes < (size_t)INT32_MAX &&
+                         imh::stream_scratch_optional(stream, 0, a_bytes + gsum_bytes + szt_bytes, &scr);
+    if (!has_szt) {
+        rc = imh::stream_scratch(stream, 0, a_bytes + (size_t)M * G * sizeof(float), &scr);
+        if (rc) return rc;
+    }
+    uint8_t *aop = static_cast<uint8_t *>(scr);
+    float *gsum = reinterpret_cast<float *>(aop + a_bytes);
+    u32x2_t *szt = reinterpret_cast<u32x2_t *>(aop + a_bytes + gsum_bytes);
+    float *part = nullptr;
+    if (splits > 1) {
+        void *p = nullptr;
+        rc = imh::stream_scratch(stream, 2, (size_t)splits * M * N * sizeof(float), &p);
+        if (rc) return rc;
+        part = static_cast<float *>(p);
+    }
+    const __bf16 *xb = static_cast<const __bf16 *>(x);
+    const __half *awq = reinterpret_cast<const __half *>(w->awq_scales);
+    const size_t chunks = (size_t)M * K / 8;
+    const int ablocks = (int)((chunks + 255) / 256);
+    const dim3 pgrid((unsigned)(ablocks + (has_szt ? ((N + 63) / 64) * ((G + 15) / 16) : 0)));
+    const dim3 grid((unsigned)(tiles * splits));
     __bf16 *out = static_cast<__bf16 *>(y);
-    if (P == PREC_BF16)
-        hipLaunchKernelGGL(gemm_mx_kernel<PREC_BF16>, grid, dim3(kThreads), 0, stream->stream, aop, gsum, w->data, sc, zr,
-                           out, part, (int)M, N, K, per, order);
-    else
-        hipLaunchKernelGGL(gemm_mx_kernel<PREC_FP8>, grid, dim3(kThreads), 0, stream->stream, aop, gsum, w->data, sc, zr,
-                           out, part, (int)M, N, K, per, order);
+#define IMH_MX(PR, MI, SZ)                                                                                              \
+    hipLaunchKernelGGL((gemm_mx_kernel<PR, MI, SZ>), grid, dim3(kThreads), 0, stream->stream, aop, gsum, w->data, w->scales, \
+                       w->zeros, szt, out, part, (int)M, N, K, per, order)
+#define IMH_MX_ALL(PR)                                                                                               \
+    hipLaunchKernelGGL(gemm_mx_prep_kernel<PR>, pgrid, dim3(256), 0, stream->stream, xb, awq, aop, gsum, chunks, K,   \
+                       ablocks, w->scales, w->zeros, szt, N);                                                        \
+    IMH_HIP(hipGetLastError());                                                                                      \
+    if (has_szt) {                                                                                                   \
+        if (bm == 32) IMH_MX(PR, 1, true);                                                                           \
+        else IMH_MX(PR, 2, true);                                                                                    \
+    } else {                                                                                                         \
+        if (bm == 32) IMH_MX(PR, 1, false);                                                                          \
+        else IMH_MX(PR, 2, false);                                                                                   \
+    }
+    if (P == PREC_BF16) {
+        IMH_MX_ALL(PREC_BF16)
+    } else {
+        IMH_MX_ALL(PREC_FP8)
+    }
+#undef IMH_MX_ALL
+#undef IMH_MX
     IMH_HIP(hipGetLastError());
     if (splits > 1) {
         const size_t count = (size_t)M * N;

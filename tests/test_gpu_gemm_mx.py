@@ -98,6 +98,39 @@ def test_gemm_mx_small(dev, stream, prec, m, n, k, awq):
     check_exact(got, operand(xb, q, prec), q, f"m={m} n={n} k={k} awq={awq}")
 
 
+@pytest.mark.parametrize("prec", [ops.GEMM_BF16, ops.GEMM_FP8_E4M3], ids=["bf16", "fp8"])
+@pytest.mark.parametrize("m,n,k,awq", [
+    (1, 31, 128, True),        # one row, one group, fewer columns than a fragment
+    (32, 257, 1152, False),    # a full 32-row tile, one column past a tile, odd group count
+    (65, 513, 384, True),      # one row past a 64-row tile
+])
+def test_gemm_mx_tile_edges(dev, stream, prec, m, n, k, awq):
+    test_gemm_mx_small(dev, stream, prec, m, n, k, awq)
+
+
+@pytest.mark.parametrize("prec", [ops.GEMM_BF16, ops.GEMM_FP8_E4M3], ids=["bf16", "fp8"])
+def test_gemm_mx_capture_reads_constants_in_place(dev, prec):
+    """Under capture with scratch for the operand rows only, scales and zero-points are read
+    in place: the replays equal the eager result bit for bit."""
+    m, k = 1024, 2048
+    q0, xb = problem(m, 256, k, 5, True)
+    q1, _ = problem(m, 8192, k, 6, True)
+    st = dev.stream()
+    xd, y0 = dev.upload(xb), dev.empty((m, 256), np.uint16)
+    ye, yg = dev.empty((m, 8192), np.uint16), dev.empty((m, 8192), np.uint16)
+    w0, w1 = ops.AffineQuantizedWeight(dev, q0), ops.AffineQuantizedWeight(dev, q1)
+    ops.encode_affine_gemm_int4(st, xd, m, w0, y0, prec)
+    g = st.capture(lambda: ops.encode_affine_gemm_int4(st, xd, m, w1, yg, prec))
+    ops.encode_affine_gemm_int4(st, xd, m, w1, ye, prec)
+    st.sync()
+    want = ye.read()
+    for _ in range(2):
+        st.zero(yg)
+        g.launch()
+        st.sync()
+        assert np.array_equal(yg.read(), want)
+
+
 @pytest.mark.parametrize("m,n,k", [(512, 9728, 2560), (512, 2560, 9728), (2048, 9728, 2560), (2048, 2560, 9728)])
 def test_gemm_mx_configs3(dev, stream, m, n, k):
     """BASELINE configs[3] at its full sizes: X bf16 N(0,1), W INT4 g128 from N(0,0.02), bf16
