@@ -29,6 +29,8 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 
 using namespace imh_wq;
 
+constexpr int kRowsMax = 32;   // rows up to which the one-launch kernel runs
+
 // Sum the split partials in split order, then store (or, for a gate/up pair,
 // apply the activation): grid ceil(M*N / 256), block 256.
 __global__ void __launch_bounds__(256) int4_gemm_reduce_kernel(const float *__restrict__ part, int splits,
@@ -133,13 +135,35 @@ __global__ void __launch_bounds__(256) resnorm_rows_kernel(const __half *__restr
 
 namespace imh_int4 {
 
+// K splits of the one-launch kernel: a split takes whole blocks of groups; a
+// round of workgroups (two per CU) costs ~4 us and ~1.05 per group, a split
+// ~3 us of reduction and its partials' round trip.  Measured at 12 rows, AWQ,
+// 9728 -> 2560: 1 / 2 / 3 / 5 blocks per split 16.1 / 18.9 / 20 / 33 us.
+int rows_splits(int M, int N, int K, int nmat, int cus) {
+    const int tiles = (N + 256 / nmat - 1) / (256 / nmat), G = K / kGS;
+    int best = 1;
+    double best_us = 1e30;
+    for (int per = kRowsBlock;; per += kRowsBlock) {
+        const int sp = (G + per - 1) / per;
+        const double us = (double)(((long long)tiles * sp + 2 * cus - 1) / (2 * cus)) * (4.0 + 1.05 * std::min(per, G)) +
+                          (sp > 1 ? 3.0 + (double)sp * M * nmat * N * 8 / 4.5e6 : 0.0);
+        if (us < best_us) {
+            best_us = us;
+            best = sp;
+        }
+        if (sp == 1) break;
+    }
+    return best;
+}
+
 // K splits (whole groups each, at least 4 per split), only as many as keep
 // the grid within one round of workgroup slots (two per CU).  Each
 // workgroup costs about the same per group (kGroupUs at two per CU, ~0.6 of
 // that alone on a CU), and a split adds its partials' round trip (read back
 // by the reduce launch at ~4.5 TB/s plus ~2 us).
 int gemm_splits(int M, int N, int K, int nmat, int cus) {
-    const int bm = M <= 32 ? 32 : 64;
+    if (M <= kRowsMax) return rows_splits(M, N, K, nmat, cus);
+    const int bm = 64;
     const int tiles = ((M + bm - 1) / bm) * ((N + 256 / nmat - 1) / (256 / nmat));
     const int G = K / kGS;
     if (tiles >= 2 * cus || G < 8) return 1;
@@ -189,14 +213,31 @@ void launch_tile(hipStream_t st, const Launch &L, bool pair) {
                        L.gsum, L.mats, L.szt, L.part, L.M, L.N, L.K, L.per, L.epi, L.order)
     if constexpr (BITS == 4) {
         if (pair) {
-            if (L.M <= 32) IMH_WQ(1, true);
-            else IMH_WQ(2, true);
+            IMH_WQ(2, true);
             return;
         }
     }
-    if (L.M <= 32) IMH_WQ(1, false);
-    else IMH_WQ(2, false);
+    IMH_WQ(2, false);
 #undef IMH_WQ
+}
+
+// Up to kRowsMax rows: one launch (and the reduction of a split).
+template <int BITS>
+void launch_rows(hipStream_t st, const Launch &L, const __half *awq, bool pair) {
+    const dim3 grid((unsigned)(L.order.tiles_n * L.order.splits));
+#define IMH_ROWS(AWQ, PAIR)                                                                                       \
+    hipLaunchKernelGGL((wq_rows_kernel<BITS, AWQ, PAIR>), grid, dim3(kThreads), 0, st, L.hi, awq, L.mats, L.part, L.M, \
+                       L.N, L.K, L.per, L.epi, L.order.tiles_n)
+    if constexpr (BITS == 4) {
+        if (pair) {
+            if (awq) IMH_ROWS(true, true);
+            else IMH_ROWS(false, true);
+            return;
+        }
+    }
+    if (awq) IMH_ROWS(true, false);
+    else IMH_ROWS(false, false);
+#undef IMH_ROWS
 }
 
 // The activation planes (with awq or INT8), transposed column constants where
@@ -206,7 +247,7 @@ int encode_wq_gemm(imh_stream *s, const __half *x, int M, const Mats &mats, cons
                    int epi, void *workspace, bool *used) {
     const int cus = s->dev->props.multiProcessorCount;
     const int G = K / kGS;
-    int splits = gemm_splits(M, N, K, nmat, cus);
+    int splits = workspace ? gemm_splits(M, N, K, nmat, cus) : 1;
     const int per = (G + splits - 1) / splits;
     splits = (G + per - 1) / per;
     Launch L = {};
@@ -218,8 +259,7 @@ int encode_wq_gemm(imh_stream *s, const __half *x, int M, const Mats &mats, cons
     L.per = per;
     L.epi = epi;
     L.part = splits == 1 ? nullptr : static_cast<float *>(workspace);
-    if (splits > 1 && !L.part) return imh::fail(IMH_EINVAL, "int4 gemm: split-K workspace missing");
-    const int bm = M <= 32 ? 32 : 64, tn = 256 / nmat;
+    const int bm = 64, tn = 256 / nmat;
     L.order.tiles_m = (M + bm - 1) / bm;
     L.order.tiles_n = (N + tn - 1) / tn;
     L.order.splits = splits;
@@ -232,7 +272,9 @@ int encode_wq_gemm(imh_stream *s, const __half *x, int M, const Mats &mats, cons
             break;
         }
     const bool pair = nmat == 2;
-    if (BITS == 4 && !awq) {
+    if (M <= kRowsMax) {
+        launch_rows<BITS>(s->stream, L, awq, pair);
+    } else if (BITS == 4 && !awq) {
         launch_tile<4, 1, true, false>(s->stream, L, pair);
     } else {
         const size_t mk = (size_t)M * K;

@@ -315,7 +315,8 @@ int run_gemm(imh_stream *s, const ActIn &in, int M, const imh_affine_int4_weight
     void *ws = nullptr;
     const size_t ws_bytes = gemm_workspace_bytes(M, N, K, nmat, cus);
     int rc = IMH_OK;
-    if (ws_bytes) {
+    // a capturing stream whose scratch lacks the partials runs the GEMM unsplit
+    if (ws_bytes && !(s->capturing && s->scratch_bytes[2] < ws_bytes)) {
         rc = imh::stream_scratch(s, 2, ws_bytes, &ws);
         if (rc) return rc;
     }
@@ -426,6 +427,20 @@ int run_matvec(imh_stream *s, ActIn in, uint32_t B, int nmat, int epi, int N, in
     return launch_image(nmat, epi, p.L, mp, in);
 }
 
+// 9 to 31 rows on the GEMM's one-launch kernel, instead of the matvec kernel's
+// 8-row passes: from ~115 M products on.  Matvec against GEMM in us: 1024 x 1024
+// at 9-31 rows 8.5 against 10-12; 3001 x 4096 at 9 / 12 / 24 rows 12.6 / 14.3 /
+// 20.9 against 13.0 / 13.4 / 14.7; 2560 x 9728 at 9 / 16 / 31 rows 23 / 33 / 43
+// against 15.5 / 16.9 / 19.5.  Only where the operand is the f16 rows as given
+// (a residual-norm source whose rows are not rounded first stays), and not when
+// a capturing stream's scratch lacks the split's partials.
+bool rows_gemm_pays(const imh_stream *s, const ActIn &in, int B, const imh_affine_int4_weight *w, int nmat) {
+    if (B < 9 || (in.b && in.round_mode != 1)) return false;
+    if ((double)B * w->n * w->k * nmat < 115e6) return false;
+    const size_t ws = gemm_workspace_bytes(B, (int)w->n, (int)w->k, nmat, s->dev->props.multiProcessorCount);
+    return !(s->capturing && s->scratch_bytes[2] < ws);
+}
+
 // Validates the weights and runs the op: x (plain) or the residual-norm
 // inputs (in.b != NULL) -> out0 [, out1].
 int run_op(imh_stream *s, ActIn in, uint32_t B, const imh_affine_int4_weight *w0,
@@ -456,7 +471,8 @@ int run_op(imh_stream *s, ActIn in, uint32_t B, const imh_affine_int4_weight *w0
     }
     mp.out[0] = reinterpret_cast<__half *>(out0);
     mp.out[1] = reinterpret_cast<__half *>(out1);
-    if ((int)B >= kGemmMinTokens) return run_gemm(s, in, (int)B, w0, w1, epi, out0, out1);
+    if ((int)B >= kGemmMinTokens || rows_gemm_pays(s, in, (int)B, w0, w1 ? 2 : 1))
+        return run_gemm(s, in, (int)B, w0, w1, epi, out0, out1);
     return run_matvec(s, in, B, w1 ? 2 : 1, epi, (int)w0->n, (int)w0->k, mp, who);
 }
 

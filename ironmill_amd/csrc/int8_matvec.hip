@@ -47,17 +47,16 @@ constexpr int kMaxWaves = 8;
 constexpr int kNG = 8;                    // groups one wave holds per stage
 constexpr int kStageBytes = 48 * 1024;    // LDS for one stage's activation
 
-// From how many batch rows the INT8 projection runs the GEMM (three launches,
-// any row count up to its tile at one cost) instead of the tile kernel (one
-// launch per 8 rows, weights read each time).  Measured, tile kernel against
-// GEMM in us: 2560 x 9728 at 5 / 8 / 16 rows 35 / 48 / 96 against 19 / 20 /
-// 20; 3001 x 4096 16.5 / 22 / 44 against 15.4 / 15.4 / 16.3; 1024 x 1024
-// 6.4 / 8.0 / 16 against 13 / 13 / 13.5 (equal at 12).  At 4 rows only what
-// the band kernel's LDS cannot hold comes here.
+// From how many batch rows the INT8 projection runs the GEMM (up to 32 rows one
+// launch and a reduction) instead of the tile kernel (one launch per 8 rows,
+// weights read each time).  Measured, tile kernel against GEMM in us: 2560 x
+// 9728 at 5 / 8 / 16 rows 35 / 48 / 95 against 17.5 / 18.5 / 18.7; 3001 x 4096
+// 16.2 / 22 / 44 against 14.1 / 14.1 / 14.9; 1024 x 1024 at 5 / 8 / 16 rows 6.4
+// / 8.0 / 16 against ~11.  At 4 rows only what the band kernel's LDS cannot
+// hold comes here.
 bool int8_gemm_pays(uint32_t rows, int N, int K) {
     if (rows > 65535) return false;
-    const long long weights = (long long)N * K;
-    return rows >= 13 || (rows >= 9 && weights >= 2000000) || (rows >= 4 && weights >= 10000000);
+    return rows >= 9 || (rows >= 4 && (long long)N * K >= 10000000);
 }
 constexpr float kTwoM24 = 5.9604644775390625e-08f;
 constexpr float kTwo24 = 16777216.0f;

@@ -46,6 +46,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
+#include "dpp_reduce.h"
 #include "imh_internal.h"
 
 namespace imh_wq {
@@ -510,6 +511,240 @@ __global__ void __launch_bounds__(kThreads, 2) wq_gemm_kernel(const __half *__re
                 }
             }
         }
+}
+
+// Up to 32 rows in one launch: bound by memory latency and launches, not by
+// any rate, so the activation's division and hi / lo split, the group sums and
+// the scale reads are part of the launch, and a workgroup has the loads of a
+// whole block of groups in flight before its first product (each wave 64
+// columns, as above; one 32-row tile).  A group's registers are loaded again, a
+// block on, as soon as it is done.  AWQ: x / awq in two planes; without, x in
+// one (INT8's second plane would be zero).  A group costs a workgroup about
+// 1.05 us on top of ~4 (one wave per SIMD issues the expansion at half rate);
+// 16 x 16 products, and eight waves with the groups halved between them, came
+// to the same or more (33 and 43 us for the FFN at 12 rows against 33).
+constexpr int kRowsBlock = 4;   // groups per block (INT8: half, for its code bytes)
+template <int BITS, bool AWQ, bool PAIR>
+__global__ void __launch_bounds__(kThreads, 2) wq_rows_kernel(const __half *__restrict__ x,
+                                                              const __half *__restrict__ awq, Mats mats,
+                                                              float *__restrict__ part, int M, int N, int K, int per,
+                                                              int epi, int tiles_n) {
+    constexpr int NPL = AWQ ? 2 : 1;
+    constexpr int TN = PAIR ? 128 : 256;
+    constexpr int PB = BITS == 8 ? kRowsBlock / 2 : kRowsBlock;
+    constexpr int WQ = BITS / 2;                     // code quads (16 bytes) per fragment and group
+    constexpr int PLANE = 8 * kBlk;
+    __shared__ __attribute__((aligned(16))) uint8_t As[PB][NPL][PLANE];
+    __shared__ __attribute__((aligned(16))) float Rs[PB][BITS == 8 ? 32 : 4];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int nl = lane & 31, h = lane >> 5;
+    const int nt = blockIdx.x % tiles_n, split = blockIdx.x / tiles_n;
+    const int nb = nt * TN;
+    const int n0 = nb + wave * (TN / 4);
+    const int G = K / kGS;
+    const int g_begin = split * per;
+    const int g_end = min(g_begin + per, G);
+
+    const int row_bytes = K * BITS / 8;
+    const int cols = min(TN, N - nb);
+    __amdgpu_buffer_rsrc_t w_r[2], s_r[2], z_r[2];
+    int bvo[2], svo[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int t = PAIR ? j : 0;
+        w_r[j] = __builtin_amdgcn_make_buffer_rsrc((void *)(mats.data[t] + (size_t)nb * row_bytes), 0,
+                                                   cols * row_bytes, kRsrcWord3);
+        s_r[j] = __builtin_amdgcn_make_buffer_rsrc((void *)(mats.scales[t] + (size_t)nb * G), 0, cols * G * 2, kRsrcWord3);
+        z_r[j] = __builtin_amdgcn_make_buffer_rsrc((void *)(mats.zeros[t] + (size_t)nb * G), 0, cols * G * 2, kRsrcWord3);
+        const int n = min(n0 + (PAIR ? 0 : 32 * j) + nl, N - 1) - nb;
+        bvo[j] = n * row_bytes + (BITS == 4 ? 32 : 64) * h;
+        svo[j] = n * G * 2;
+    }
+    u32x4_t bw[PB][2][WQ];
+    uint16_t bs[PB][2], bz[PB][2];
+    auto load_b = [&](int i, int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+#pragma unroll
+            for (int q = 0; q < WQ; q++)
+                bw[i][j][q] = __builtin_bit_cast(
+                    u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(w_r[j], bvo[j] + 16 * q, g * (kGS * BITS / 8), 0));
+            bs[i][j] = __builtin_amdgcn_raw_buffer_load_b16(s_r[j], svo[j], g * 2, 0);
+            bz[i][j] = __builtin_amdgcn_raw_buffer_load_b16(z_r[j], svo[j], g * 2, 0);
+        }
+    };
+    // the activation: rows tid / 16 and + 16, chunk tid % 16 of each group (rows past M read as zeros)
+    const __amdgpu_buffer_rsrc_t x_r = __builtin_amdgcn_make_buffer_rsrc((void *)x, 0, M * K * 2, kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t q_r =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(AWQ ? awq : x), 0, K * 2, kRsrcWord3);
+    const int ar0 = tid >> 4, ac = tid & 15;
+    const int xvo = (ar0 * K + ac * 8) * 2;
+    const bool two = M > 16;
+    const int a_lds = (ac & 7) * kBlk + (ar0 + 32 * (ac >> 3)) * 16;
+    u32x4_t xr[PB][2], qr[PB];
+    auto load_x = [&](int g0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PB; i++) {
+            const int g = min(g0 + i, g_end - 1);
+            if (AWQ) qr[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(q_r, ac * 16, g * 256, 0));
+            xr[i][0] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_r, xvo, g * 256, 0));
+            if (two) xr[i][1] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_r, xvo, g * 256 + 32 * K, 0));
+        }
+    };
+    constexpr int kSlot4[8] = {0, 4, 1, 5, 2, 6, 3, 7};
+    auto store_x = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PB; i++) {
+            const _Float16 *qh = reinterpret_cast<const _Float16 *>(&qr[i]);
+            float inv[8];
+            if (AWQ) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) inv[e] = __builtin_amdgcn_rcpf((float)qh[e]);
+            }
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                half8_t hi = {}, lo = {};   // rows 16-31 of a call with fewer: zeros
+                float sum = 0.0f;
+                if (p == 0 || two) {
+                    const _Float16 *xh = reinterpret_cast<const _Float16 *>(&xr[i][p]);
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        const int e = BITS == 4 ? kSlot4[k] : k;
+                        const float v = AWQ ? (float)xh[e] * inv[e] : (float)xh[e];
+                        hi[k] = (_Float16)v;
+                        lo[k] = (_Float16)(v - (float)hi[k]);
+                        if (BITS == 8) sum += (float)hi[k] + (AWQ ? (float)lo[k] : 0.0f);
+                    }
+                }
+                *reinterpret_cast<half8_t *>(&As[i][0][a_lds + p * 256]) = hi;
+                if (AWQ) *reinterpret_cast<half8_t *>(&As[i][NPL - 1][a_lds + p * 256]) = lo;
+                if (BITS == 8) {   // a row's 16 chunks are 16 consecutive lanes
+                    sum = imh_dpp::row16_sum(sum);
+                    if (ac == 0) Rs[i][ar0 + 16 * p] = sum * kTwoM24;
+                }
+            }
+        }
+    };
+
+    uint32_t m_lo, m_hi, exp1k;
+    asm("s_mov_b32 %0, 0x000f000f" : "=s"(m_lo));
+    asm("s_mov_b32 %0, 0x00f000f0" : "=s"(m_hi));
+    asm("v_mov_b32 %0, 0x64006400" : "=v"(exp1k));
+    float16_t acc[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[j][i] = 0.0f;
+    auto compute = [&](int i) __attribute__((always_inline)) {
+        float sc[2], nz[2];
+        uint32_t b1[2], b16[2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const u32x2_t c = column_consts<BITS>(bs[i][j], bz[i][j]);
+            const uint32_t cs = c[0], cz = c[1];   // scalars: a bit cast of a vector element takes element 0
+            sc[j] = __builtin_bit_cast(float, cs);
+            nz[j] = __builtin_bit_cast(float, cz);
+            b1[j] = __builtin_amdgcn_perm(cz, cz, 0x01000100u);
+            b16[j] = __builtin_amdgcn_perm(cz, cz, 0x03020302u);
+        }
+        const float16_t zero16 = {};
+        float16_t gg[2];
+        const uint8_t *ab = &As[i][0][lane * 16];
+#pragma unroll
+        for (int st = 0; st < 8; st++) {
+            half8_t af[NPL], bf[2];
+#pragma unroll
+            for (int p = 0; p < NPL; p++) af[p] = *reinterpret_cast<const half8_t *>(ab + p * PLANE + st * kBlk);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                u32x4_t o;
+                if (BITS == 4) {
+                    const uint32_t w = bw[i][j][(st >> 2) % WQ][st & 3], w8 = w >> 8;
+                    const half2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
+                    o[0] = as_u32(as_h2((w & m_lo) | exp1k) + as_h2(b1[j]));
+                    o[1] = as_u32(__builtin_elementwise_fma(as_h2((w & m_hi) | exp1k), sixteenth, as_h2(b16[j])));
+                    o[2] = as_u32(as_h2((w8 & m_lo) | exp1k) + as_h2(b1[j]));
+                    o[3] = as_u32(__builtin_elementwise_fma(as_h2((w8 & m_hi) | exp1k), sixteenth, as_h2(b16[j])));
+                } else {
+                    const uint32_t w0 = bw[i][j][(st >> 1) % WQ][2 * (st & 1)], w1 = bw[i][j][(st >> 1) % WQ][2 * (st & 1) + 1];
+                    o[0] = __builtin_amdgcn_perm(0u, w0, 0x0C010C00u);
+                    o[1] = __builtin_amdgcn_perm(0u, w0, 0x0C030C02u);
+                    o[2] = __builtin_amdgcn_perm(0u, w1, 0x0C010C00u);
+                    o[3] = __builtin_amdgcn_perm(0u, w1, 0x0C030C02u);
+                }
+                bf[j] = __builtin_bit_cast(half8_t, o);
+            }
+#pragma unroll
+            for (int p = 0; p < NPL; p++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    gg[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[p], bf[j], st == 0 && p == 0 ? zero16 : gg[j], 0, 0, 0);
+        }
+        float4_t rs[4];
+        if (BITS == 8) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) rs[q] = *reinterpret_cast<const float4_t *>(&Rs[i][8 * q + 4 * h]);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                float v = gg[j][k];
+                if (BITS == 8) v = __builtin_fmaf(nz[j], rs[k >> 2][k & 3], v);
+                acc[j][k] = __builtin_fmaf(sc[j], v, acc[j][k]);
+            }
+    };
+
+    if (g_begin < g_end) {
+        load_x(g_begin);
+#pragma unroll
+        for (int i = 0; i < PB; i++) load_b(i, min(g_begin + i, g_end - 1));
+        __builtin_amdgcn_sched_barrier(0);   // every load above issues before the first wait
+    }
+    for (int g0 = g_begin; g0 < g_end; g0 += PB) {
+        store_x();
+        __syncthreads();
+        const bool more = g0 + PB < g_end;
+        if (more) load_x(g0 + PB);
+#pragma unroll
+        for (int i = 0; i < PB; i++) {
+            if (g0 + i < g_end) compute(i);
+            if (more) load_b(i, min(g0 + PB + i, g_end - 1));
+        }
+        if (more) __syncthreads();   // the planes are rewritten next
+    }
+
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int m = 8 * (i >> 2) + 4 * h + (i & 3);
+        if (m >= M) continue;
+        if (PAIR) {
+            const int n = n0 + nl;
+            if (n >= N) continue;
+            const float g = acc[0][i], u = acc[1][i];
+            if (part) {
+                float *p = part + ((size_t)split * M + m) * 2 * N + n;
+                p[0] = g;
+                p[N] = u;
+            } else if (epi == GE_STORE) {
+                mats.out[0][(size_t)m * N + n] = __float2half(g);
+                mats.out[1][(size_t)m * N + n] = __float2half(u);
+            } else {
+                mats.out[0][(size_t)m * N + n] = __float2half(gate_act(g, u, epi));
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int n = n0 + 32 * j + nl;
+                if (n >= N) continue;
+                if (part) part[((size_t)split * M + m) * N + n] = acc[j][i];
+                else mats.out[0][(size_t)m * N + n] = __float2half(acc[j][i]);
+            }
+        }
+    }
 }
 
 }  // namespace imh_wq

@@ -214,6 +214,42 @@ def test_gemm_tile_edges(dev, stream, m, n, k, awq):
     assert np.all(err <= bound), f"m={m} n={n} k={k} awq={awq}: worst {np.max(err / bound):.2f} of the bound"
 
 
+@pytest.mark.parametrize("m,n,k,awq", [
+    (9, 12801, 1024, True),    # the fewest rows, one column past a tile, two blocks of groups
+    (16, 7001, 1152, False),   # a full half tile, an odd group count, unsplit and split blocks
+    (17, 6007, 1152, True),    # one row into the second half
+    (31, 2560, 9728, True),    # split K
+])
+def test_gemm_rows_kernel(dev, stream, m, n, k, awq):
+    """The one-launch kernel of 9 to 31 rows, to test_gemm_tile_edges' bound."""
+    assert m * n * k >= 115e6
+    test_gemm_tile_edges(dev, stream, m, n, k, awq)
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+def test_gemm_rows_gate_up(dev, stream, act):
+    """Gate and up of 12 rows in one launch, both epilogues: within 2 f16 steps of the exact
+    value plus test_gemm_fused_gate_up's slack."""
+    m, n, k = 12, 5121, 1024
+    wg, s = weight(n, k, 141, True)
+    wu, _ = weight(n, k, 142, False)
+    x16 = acts(m, k, 143)
+    qg, qu = quant.quantize_int4(wg, awq_scales=s), quant.quantize_int4(wu, awq_scales=s)
+    out = dev.empty((m, n), np.float16)
+    ops.encode_fused_ffn_gate_up_act_int4(stream, dev.upload(x16), ops.AffineQuantizedWeight(dev, qg),
+                                          ops.AffineQuantizedWeight(dev, qu), out, m, use_gelu=(act == "gelu"))
+    stream.sync()
+    xa = x16.astype(np.float64) / s.astype(np.float16).astype(np.float64)
+    Wg, Wu = exact_weights(qg), exact_weights(qu)
+    g, u = xa @ Wg.T, xa @ Wu.T
+    mg, mu = np.abs(xa) @ np.abs(Wg).T, np.abs(xa) @ np.abs(Wu).T
+    a = g / (1.0 + np.exp(-g)) if act == "silu" else 0.5 * g * (1.0 + np.tanh(0.7978845608028654 * (g + 0.044715 * g ** 3)))
+    bound = 2.0 * np.spacing(np.abs(a * u).astype(np.float16)).astype(np.float64) \
+        + 2.0 ** -16 * 1.1 * (np.abs(u) * mg + np.abs(a) * mu)
+    err = np.abs(out.read().astype(np.float64) - a * u)
+    assert np.all(err <= bound), f"worst {np.max(err / bound):.2f} of the bound"
+
+
 def test_gemm_capture_reads_constants_in_place(dev):
     """Under capture with scratch for the activation planes only, the GEMM reads scales and
     zero-points in place: the replays equal the eager result bit for bit."""
@@ -236,3 +272,25 @@ def test_gemm_capture_reads_constants_in_place(dev):
         g.launch()
         st.sync()
         assert np.array_equal(yg.read().view(np.uint16), want)
+
+
+@pytest.mark.parametrize("m", [32, 40])
+def test_gemm_capture_without_partials(dev, m):
+    """A capture on a stream without room for split partials runs the GEMM unsplit: each replay
+    is within 2 f16 steps plus the sum-order slack of the exact value."""
+    n, k = 1000, 4096
+    w, _ = weight(n, k, 151, False)
+    q = quant.quantize_int4(w)
+    x16 = acts(m, k, 152)
+    st = dev.stream()
+    xd, y, wt = dev.upload(x16), dev.empty((m, n), np.float16), ops.AffineQuantizedWeight(dev, q)
+    g = st.capture(lambda: ops.encode_projection(st, xd, wt, y, m))
+    W = exact_weights(q)
+    exact = x16.astype(np.float64) @ W.T
+    bound = 2.0 * np.spacing(np.abs(exact).astype(np.float16)).astype(np.float64) \
+        + 2.0 ** -16 * (np.abs(x16.astype(np.float64)) @ np.abs(W).T)
+    for _ in range(2):
+        st.zero(y)
+        g.launch()
+        st.sync()
+        assert np.all(np.abs(y.read().astype(np.float64) - exact) <= bound)

@@ -85,7 +85,8 @@ def test_int8_projection(dev, stream, n, k, b, awq):
 
 
 @pytest.mark.parametrize("n,k,b,awq", [
-    (256, 128, 13, False),     # GEMM: one group, one plane, one 32-row tile
+    (256, 128, 9, False),      # GEMM: one group, one plane, fewer than 16 rows
+    (1000, 1152, 17, True),    # an odd group count, one row into the second half
     (1000, 1024, 32, True),    # ragged N, a full 32-row tile
     (1000, 1024, 33, True),    # 64-row tiles, the first row of the second half
     (257, 1152, 65, False),    # one column and one row past a tile, odd group count
