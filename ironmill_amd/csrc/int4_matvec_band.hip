@@ -638,8 +638,8 @@ bool launch_shape(int tm, int bm, int xc, const BandLaunch &L, const MatPtrs &mp
 
 // Launches the band kernel when it applies (B <= 8, no row segments, an even
 // number of groups, the shape within the instantiated tiles and the LDS
-// budget -- 64 KB for 1-2 batch rows, 160 KB with one activation chunk per
-// thread above; an operand image source (in.img_src, 1-2 batch rows) or
+// budget of 160 KB, with one activation chunk per thread above 2 rows; an
+// operand image source (in.img_src, 1-2 batch rows) or
 // output (in.img_out_hi, every band on even rows); a
 // residual-norm source only at 1-2 batch rows, with
 // round_mode 0 or 1, as nmat 1 with EPI_STORE or nmat 2 with an activation);
@@ -672,7 +672,12 @@ int launch_band_matvec(hipStream_t st, int cus, int B, int nmat, int epi, int N,
     // tall matrices at 1-2 rows (the LM head): bands of 3 tiles, two waves of
     // five pairs each -- 37.5 against 38.4 us with 5-tile bands of four waves
     // (151936 x 2560 at one row, A/B on one box)
-    const bool tall12 = bm <= 2 && nmat == 1 && (ntiles + 4) / 5 > cus;
+    // and, without a norm to redo, what 5-tile bands of eight waves of three
+    // pairs cannot hold (K > 6144): tile kernel against these bands in us at 1 /
+    // 2 rows: 8192 x 8192 15.3 / 23.7 against 10.6 / 13.5, 6200 x 6400 11.1 /
+    // 15.7 against 9.2 / 12.0 (with the norm 12.3 / 18.5 against 13.6 / 21.3)
+    const bool tall12 = bm <= 2 && nmat == 1 &&
+                        ((ntiles + 4) / 5 > cus || (!rn && P > 24 && ntiles > 3 * cus));
     const int nwg = mb ? cus : std::min(std::max(cus, tall12 ? (ntiles + 2) / 3 : (ntiles + 4) / 5), N);
     if ((uint64_t)N * nwg >= (1ull << 32)) return IMH_OK;
     const int rows = mb ? 40 : (N + nwg - 1) / nwg;   // mb: rows per block
@@ -707,7 +712,10 @@ int launch_band_matvec(hipStream_t st, int cus, int B, int nmat, int epi, int N,
     const int xc = (G * 16 + nthr - 1) / nthr;
     if (xc > 3 || (bm > 2 && xc > 1) || nmat * rows * P > kSZC * nthr) return IMH_OK;
     const size_t lds = band_lds(G, bm, nmat, TM, W * nmat, rn).total;
-    if (lds > (bm <= 2 ? 64 : 160) * 1024) return IMH_OK;
+    // the operand image of 2 rows passes 64 KB from K ~ 7000: prep + tile kernel
+    // against one band launch 12.8 -> 8.0 us (2560 x 9728), 13.0 -> 7.0 (1024 x
+    // 8192), 75.9 -> 33.1 (28672 x 8192); with the norm 17.6 -> 11.7 (2560 x 9728)
+    if (lds > 160 * 1024) return IMH_OK;
     // a probe takes the same dispatch with launches off: the instantiation
     // must still accept its LDS size (hipFuncSetAttribute above 64 KB)
     // the leading arguments (see int4_band_kernel) and the packed dimensions

@@ -318,3 +318,43 @@ def test_error_paths(dev, stream):
         ops.encode_fused_ffn_gate_up_act_int4(stream, xd, wt, other, yd, 1)
     ops.encode_projection(stream, xd, wt, yd, 0)  # zero tokens: no-op
     stream.sync()
+
+
+def random_int4(n, k, seed):
+    """Random codes, scales, zero-points and AWQ scales, and the exact weights (64-bit)."""
+    rng = np.random.default_rng(seed)
+    data = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    scales = rng.uniform(0.001, 0.003, (n, k // 128)).astype(np.float16)
+    zeros = rng.integers(0, 16, (n, k // 128)).astype(np.float16)
+    awq = rng.uniform(0.5, 2.0, k).astype(np.float16)
+    q = quant.QuantizedInt4(data=data, scales=scales, zeros=zeros, scales_f32=None, zeros_f32=None, awq=awq, n=n, k=k)
+    codes = np.empty((n, k), np.float64)
+    codes[:, 0::2], codes[:, 1::2] = data & 15, data >> 4
+    z = np.repeat(zeros.astype(np.float64), 128, 1)
+    return q, (codes - z) * np.repeat(scales.astype(np.float64), 128, 1), awq.astype(np.float64)
+
+
+# The balanced band kernel past 64 KB of operand image (2 rows), at its most groups
+# (80), and with the 3-tile bands of many rows and more than 48 groups, ragged or not.
+# Bound: 2 f16 steps, plus 2^-16 of the magnitude sum for the f32 sums and the hi + lo
+# split of x / awq (22 bits, against raw codes of up to 15 per unit of q - z).
+@pytest.mark.parametrize("n,k,batch", [
+    (300, 9728, 2), (513, 10240, 2), (6401, 6400, 1), (6401, 6400, 2), (6150, 10240, 2),
+])
+def test_band_wide_operands(dev, stream, n, k, batch):
+    q, W, awq = random_int4(n, k, n + batch)
+    x16 = make_x(batch, k, seed=n)
+    y = dev.empty((batch, n), np.float16)
+    ops.encode_projection(stream, dev.upload(x16), ops.AffineQuantizedWeight(dev, q), y, batch)
+    stream.sync()
+    xa = x16.astype(np.float64) / awq
+    exact = xa @ W.T
+    bound = 2.0 * np.spacing(np.abs(exact).astype(np.float16)).astype(np.float64) \
+        + 2.0 ** -16 * (np.abs(xa) @ np.abs(W).T)
+    err = np.abs(y.read().astype(np.float64) - exact)
+    assert np.all(err <= bound), f"worst {np.max(err / bound):.2f} of the bound"
+
+
+@pytest.mark.parametrize("n,k", [(256, 9728), (6401, 6400)])
+def test_band_wide_residual_norm(dev, stream, n, k):
+    test_fused_residual_norm_projection(dev, stream, n, k, 2, True)
