@@ -893,17 +893,94 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 // consecutive tokens x the GQA heads: a KV chunk's codes are looked up once
 // for all of them, the partial products go to separate MFMAs (20 per chunk
 // instead of 12 per token), and P.V fills every row.
-//   * launch_tq_query_prep rotates each query row, projects it onto the QJL
-//     matrix in f32 and stores the four f16 operand planes q_hi, q_lo, s_hi,
-//     s_lo in MFMA k-slot order;
+//   * tq_query_prep_rows_kernel rotates each query row, projects it onto the
+//     QJL matrix (the decode prologue's arithmetic, same f32 order) and
+//     stores the four f16 operand planes q_hi, q_lo, s_hi, s_lo in MFMA
+//     k-slot order;
 //   * tq_prefill_attention_kernel<GQA>, one workgroup per (split, kv head,
 //     token block of a sequence), keeps a per-row online softmax; each row
 //     has its own causal bound (turboquant.metal:268);
-//   * with several splits, launch_prefill_combine merges the partials
+//   * with several splits, a combine launch merges the partials
 //     (log-sum-exp, fused_sdpa_reduce, flash_decode.metal:163-215) and
 //     rotates back; with one, the attention kernel does.
 // ---------------------------------------------------------------------------
 constexpr int kQPlanes = 4;   // q_hi, q_lo, s_hi, s_lo, kD halfs each
+
+// element p of an operand plane holds dimension (p & ~7) | slot(p & 7): the
+// k-slot order {0, 2, 1, 3, 4, 6, 5, 7} of the code-byte unpack (bits 0 and 1
+// swapped)
+__device__ __forceinline__ int plane_dim(int p) { return (p & ~7) | ((p & 1) << 1) | ((p >> 1) & 1) | (p & 4); }
+
+// grid ceil(rows / 4), block 256: wave w rotates query row 4 blockIdx.x + w
+// (rows = batch x tokens x heads, [row][kD] f16), then the workgroup projects
+// its four rows and writes their planes ([row][kQPlanes][kD] f16).  For the
+// token blocks' few rows: 512 / 752 / 2048 rows 4.2 / 5.2 / 6.4 us against 7.4 /
+// 7.6 / 9.0 of launch_tq_query_prep's 32-row workgroups (16384 rows 18.9 : 17.8).
+__global__ void __launch_bounds__(256) tq_query_prep_rows_kernel(const __half *__restrict__ q, int rows,
+                                                            const float *__restrict__ signs,
+                                                            const float *__restrict__ qjl_t,
+                                                            _Float16 *__restrict__ planes) {
+    __shared__ float qs[4][2][kD];
+    __shared__ float om[4][4][kD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row0 = blockIdx.x * 4;
+    const int kr = tid >> 5, dq = tid & 31;
+    const float rscale = 1.0f / sqrtf((float)kD);
+    const __half *qh = q + (size_t)min(row0 + wave, rows - 1) * kD;
+    const float sg0 = signs[lane], sg1 = signs[lane + 64];
+    float x0 = __half2float(qh[lane]) * sg0, x1 = __half2float(qh[lane + 64]) * sg1;
+    float4 st[16];
+    {
+        const float4 *s4 = reinterpret_cast<const float4 *>(qjl_t) + (size_t)kr * 16 * (kD / 4) + dq;
+#pragma unroll
+        for (int i = 0; i < 16; i++) st[i] = s4[(size_t)i * (kD / 4)];
+    }
+    x0 = hadamard64(x0, lane);
+    x1 = hadamard64(x1, lane);
+    qs[wave][0][lane] = (x0 + x1) * (sg0 * rscale);
+    qs[wave][0][lane + 64] = (x0 - x1) * (sg1 * rscale);
+    __syncthreads();
+    float4 pr[4];
+#pragma unroll
+    for (int hh = 0; hh < 4; hh++) pr[hh] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+#pragma unroll
+        for (int hh = 0; hh < 4; hh++) {
+            const float qv = qs[hh][0][kr * 16 + i];
+            pr[hh].x = __builtin_fmaf(st[i].x, qv, pr[hh].x);
+            pr[hh].y = __builtin_fmaf(st[i].y, qv, pr[hh].y);
+            pr[hh].z = __builtin_fmaf(st[i].z, qv, pr[hh].z);
+            pr[hh].w = __builtin_fmaf(st[i].w, qv, pr[hh].w);
+        }
+    }
+#pragma unroll
+    for (int hh = 0; hh < 4; hh++) {
+        pr[hh].x += __shfl_xor(pr[hh].x, 32);
+        pr[hh].y += __shfl_xor(pr[hh].y, 32);
+        pr[hh].z += __shfl_xor(pr[hh].z, 32);
+        pr[hh].w += __shfl_xor(pr[hh].w, 32);
+        if (lane < 32) reinterpret_cast<float4 *>(&om[wave][hh][0])[dq] = pr[hh];
+    }
+    __syncthreads();
+    for (int e = tid; e < 4 * kD; e += 256) {
+        const int hh = e / kD, d = e % kD;
+        qs[hh][1][d] = (om[0][hh][d] + om[1][hh][d]) + (om[2][hh][d] + om[3][hh][d]);
+    }
+    __syncthreads();
+    for (int e = tid; e < 4 * kD; e += 256) {
+        const int hh = e / kD, p = e % kD;
+        if (row0 + hh >= rows) continue;
+        const int d = plane_dim(p);
+        const float vq = qs[hh][0][d], vs = qs[hh][1][d];
+        const _Float16 qhi = (_Float16)vq, shi = (_Float16)vs;
+        _Float16 *dst = planes + (size_t)(row0 + hh) * kQPlanes * kD + p;
+        dst[0] = qhi;
+        dst[kD] = (_Float16)(vq - (float)qhi);
+        dst[2 * kD] = shi;
+        dst[3 * kD] = (_Float16)(vs - (float)shi);
+    }
+}
 
 // grid (S, nkv, batch x ceil(T / TB)), block 256; TB = 16 / GQA tokens per
 // workgroup.  MFMA row r = TB-local token r / GQA, head r % GQA; lane (n, g)
@@ -1119,11 +1196,12 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 }
 
 // grid rows, block 256: one workgroup merges the S split partials of its row
-// ([row][S] maxima and sums, [row][S][kD] outputs) and rotates the result
-// back into out[row].  Split s weighs exp(m_s - M); wave w sums the splits
+// ([row][S] maxima -- LOG2: in log2 units, from the prefill kernel -- and sums,
+// [row][S][kD] outputs) and rotates the result back into out[row].  Split s weighs exp(m_s - M); wave w sums the splits
 // w, w + 4, .. (the first sixteen of them loaded together with the maxima), the
 // four partial sums are added in wave order through LDS, and wave 0
 // normalises and rotates.
+template <bool LOG2>
 __global__ void __launch_bounds__(256) tq_split_combine_kernel(const float *__restrict__ part_o,
                                                                const float *__restrict__ part_m,
                                                                const float *__restrict__ part_l, int rows, int S,
@@ -1155,7 +1233,8 @@ __global__ void __launch_bounds__(256) tq_split_combine_kernel(const float *__re
     for (int st = 32; st >= 1; st >>= 1) mx = fmaxf(mx, __shfl_xor(mx, st));
     float o0 = 0.0f, o1 = 0.0f, ls = 0.0f;
     auto add = [&](float m, float l, float a0, float a1) __attribute__((always_inline)) {
-        const float f = (mx == -INFINITY || m == -INFINITY) ? 0.0f : __expf(m - mx);
+        const float f = (mx == -INFINITY || m == -INFINITY) ? 0.0f
+                                                            : (LOG2 ? __builtin_amdgcn_exp2f(m - mx) : __expf(m - mx));
         ls = __builtin_fmaf(f, l, ls);
         o0 = __builtin_fmaf(a0, f, o0);
         o1 = __builtin_fmaf(a1, f, o1);
@@ -1351,9 +1430,9 @@ static int run_prefill_attention(imh_stream *stream, const imh_tq_tables *t, con
         pls = pm + rows * S;
     }
     _Float16 *planes = static_cast<_Float16 *>(pl_scr);
-    rc = imh::launch_tq_query_prep(stream, reinterpret_cast<const __half *>(q), rows, t->signs, t->qjl_t, planes);
-    if (rc) return rc;
     if (tile_kernel) {
+        rc = imh::launch_tq_query_prep(stream, reinterpret_cast<const __half *>(q), rows, t->signs, t->qjl_t, planes);
+        if (rc) return rc;
         imh::PrefillAttention a = {};
         a.q = planes;
         a.k = cache->k_codes;
@@ -1380,6 +1459,9 @@ static int run_prefill_attention(imh_stream *stream, const imh_tq_tables *t, con
         rc = imh::launch_prefill_attention(stream, true, cache->batch, S, a);
         if (rc) return rc;
     } else {
+        hipLaunchKernelGGL(tq_query_prep_rows_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream->stream,
+                           reinterpret_cast<const __half *>(q), (int)rows, t->signs, t->qjl_t, planes);
+        IMH_HIP(hipGetLastError());
         const dim3 grid(S, nkv, cache->batch * ntb);
 #define IMH_TQ_PREFILL(G)                                                                                       \
         hipLaunchKernelGGL((tq_prefill_attention_kernel<G>), grid, dim3(64 * kWaves), 0, stream->stream, planes,      \
@@ -1393,7 +1475,14 @@ static int run_prefill_attention(imh_stream *stream, const imh_tq_tables *t, con
 #undef IMH_TQ_PREFILL
         IMH_HIP(hipGetLastError());
     }
-    if (S > 1) return imh::launch_prefill_combine(stream, true, rows, S, po, pm, pls, t->signs, reinterpret_cast<__half *>(out));
+    if (S <= 1) return IMH_OK;
+    // the merge: a workgroup per row up to 1024 rows (512 / 752 rows 4.6 / 4.7 us
+    // against 6.8 / 6.0 with a wave per row), a wave per row above (2048 rows 6.7 : 4.7)
+    if (rows > 1024)
+        return imh::launch_prefill_combine(stream, true, rows, S, po, pm, pls, t->signs, reinterpret_cast<__half *>(out));
+    hipLaunchKernelGGL(tq_split_combine_kernel<true>, dim3((unsigned)rows), dim3(256), 0, stream->stream, po, pm, pls,
+                       (int)rows, (int)S, t->signs, reinterpret_cast<__half *>(out));
+    IMH_HIP(hipGetLastError());
     return IMH_OK;
 }
 
@@ -1545,7 +1634,7 @@ static int run_attention(imh_stream *stream, const imh_tq_tables *t, const imh_t
     IMH_HIP(hipGetLastError());
     if (S > 1) {   // the splits' merge, in stream order after every partial
         const int rows = (int)(B * num_heads);
-        hipLaunchKernelGGL(tq_split_combine_kernel, dim3((unsigned)rows), dim3(256), 0, stream->stream, po, pm,
+        hipLaunchKernelGGL(tq_split_combine_kernel<false>, dim3((unsigned)rows), dim3(256), 0, stream->stream, po, pm,
                            pl, rows, (int)S, t->signs, reinterpret_cast<__half *>(out));
         IMH_HIP(hipGetLastError());
     }
