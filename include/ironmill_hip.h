@@ -171,7 +171,7 @@ int imh_encode_fused_ffn_gate_up_act_int4(imh_stream *stream, const uint16_t *x,
  * f16(act(x.Wg) * (x.Wu)) as imh_encode_fused_ffn_gate_up_act_int4 writes it
  * (act_out [token_count][gate->n]), then y = act_out . Wd^T with down's
  * awq_scales (y [token_count][down->n]), with the two ops' results (matvec
- * below 32 tokens, GEMM from 32; at 1-2 tokens the gate/up launch also hands
+ * below 32 tokens, 9 for large weights, then GEMM; at 1-2 tokens the gate/up launch also hands
  * the down launch its operand image through the stream's scratch).  down->k
  * must equal gate->n. */
 int imh_encode_ffn_block_int4(imh_stream *stream, const uint16_t *x, uint32_t token_count,
@@ -182,8 +182,8 @@ int imh_encode_ffn_block_int4(imh_stream *stream, const uint16_t *x, uint32_t to
 /* Prefill GEMM at a chosen matrix-core precision (superblock_matmul_int4,
  * affine_matmul.metal:10-152, at the precisions of the prefill workload):
  *   y[m][n] = sum_k a[m][k] * (q[n][k] - z) * s,  f32 accumulate, a = x / awq.
- * IMH_GEMM_F16: x and y f16 -- the projection op above (matvec below 32
- *   tokens, the f16 GEMM from 32);
+ * IMH_GEMM_F16: x and y f16 -- the projection op above (matvec or, from 32
+ *   tokens and 9 for large weights, the f16 GEMM);
  * IMH_GEMM_BF16: x and y bf16, a rounded once to bf16, bf16 matrix cores;
  * IMH_GEMM_FP8_E4M3: x and y bf16, a rounded once to OCP e4m3 (saturating at
  *   +-448), fp8 matrix cores.
@@ -211,7 +211,9 @@ typedef struct {
 
 /* superblock_matvec_int8 (affine_matvec.metal:123-189) for token_count rows:
  * y[t][r] = f16( sum_k (x[t][k] / awq[k]) * (q[r][k] - z) * s ), f32 accumulate.
- * x [token_count][k] f16, y [token_count][n] f16. */
+ * x [token_count][k] f16, y [token_count][n] f16.  From 9 rows (4 for large
+ * weights) a GEMM over operand planes in the stream's scratch; a capture whose
+ * stream lacks that scratch records the matvec, which needs none. */
 int imh_encode_affine_projection_int8(imh_stream *stream, const uint16_t *x, uint32_t token_count,
                                       const imh_affine_int8_weight *w, uint16_t *y);
 
@@ -368,9 +370,9 @@ int imh_encode_turboquant_attention_noalloc(imh_stream *stream, const imh_tq_tab
  * [head_dim] f16; token t of sequence b attends to positions
  * [0, L_b - token_count + t + 1) with L_b as in imh_encode_turboquant_attention
  * (the length including the new tokens, whose K / V the cache already holds).
- * One workgroup serves 16 / GQA consecutive tokens x the GQA group's heads
- * (each KV chunk is read and decoded once for all of them), after a query
- * prep launch; num_splits as in imh_encode_turboquant_attention (0: automatic,
+ * After a query prep launch one workgroup serves 256 (token, head) rows of a kv
+ * head, or 16 / GQA tokens x the GQA group's heads where the rows are few (each
+ * KV chunk is read and decoded once for all of them); num_splits as in imh_encode_turboquant_attention (0: automatic,
  * over the longest causal range), with a combine launch when there are
  * several.  Uses the stream's scratch (batch x token_count x num_heads KB of
  * query operands, plus the split partials).  batch x ceil(token_count x GQA /
@@ -509,8 +511,8 @@ int imh_encode_kv_scatter(imh_stream *stream, const imh_fp16_kv_cache *cache, co
  * seq_len, 0 = max_seq_len, when seq_lens is given; out has q's layout.  A row
  * with no position gives 0.  num_splits = 0 picks the KV split count from the
  * shape.  seq_len > max_seq_len is IMH_ERANGE; token_count > seq_len (without
- * seq_lens) is IMH_EINVAL.  The kernel is built for decode (token_count 1);
- * larger token counts are computed correctly, without prefill tiling. */
+ * seq_lens) is IMH_EINVAL.  A prefill chunk runs on tiles of 128 (token,
+ * head) rows, decode and few rows on a workgroup per 4. */
 int imh_encode_fp16_attention(imh_stream *stream, const imh_fp16_kv_cache *cache, const uint16_t *q,
                               uint32_t num_heads, uint32_t token_count, uint32_t seq_len,
                               const int32_t *seq_lens, float attn_scale, uint16_t *out,

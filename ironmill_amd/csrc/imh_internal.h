@@ -42,8 +42,8 @@ struct imh_buffer {
 };
 
 // Per-stream scratch memory, grown on demand by the host code of an op.
-// Slot 0: INT4 activation operand images, the query operand planes of the
-// TurboQuant prefill attention; slot 1: attention split partials,
+// Slot 0: INT4 activation operand images, GEMM operand planes and transposed
+// scales, the query operand planes of the TurboQuant prefill attention; slot 1: attention split partials,
 // the gate output of a prefill gate/up op; slot 2: GEMM and INT4 matvec split-K partials.
 // A graph captured on the stream records the slots' addresses, so a slot that
 // grows later keeps its old block alive (`retired`) until the stream is freed:
@@ -126,7 +126,7 @@ int encode_segmented_matvec_int4(imh_stream *s, const uint16_t *x, const imh_fus
 // written as by imh_encode_fused_residual_norm_affine_matvec_int4; rn->weight
 // and rn->output are not read) feeding the fused gate + up + SiLU/GELU of
 // imh_encode_fused_ffn_gate_up_act_int4 with the f16 normed rows as its
-// input (as after a separate norm), in one launch below 32 tokens.
+// input (as after a separate norm), in one launch up to 8 tokens.
 int encode_resnorm_gate_up_act_int4(imh_stream *s, const imh_fused_residual_norm_params *rn, uint32_t B,
                                     const imh_affine_int4_weight *gate, const imh_affine_int4_weight *up,
                                     uint16_t *out, int use_gelu);

@@ -544,7 +544,7 @@ int imh_affine_gemm_int4(imh_stream *stream, const void *x, uint32_t M, const im
     int rc = check_gemm_weight(w, who);
     if (rc) return rc;
     if (precision == IMH_GEMM_F16) {
-        // the f16 path is the projection op (matvec below 32 tokens, f16 GEMM from 32)
+        // the f16 path is the projection op (matvec or f16 GEMM)
         return imh_encode_affine_projection_int4(stream, static_cast<const uint16_t *>(x), M, w,
                                                  static_cast<uint16_t *>(y));
     }
