@@ -254,10 +254,12 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_mx_kernel(
             }
         }
     };
-    // A: pass i of a thread is row RPP i + tid / CPR, chunk tid % CPR; rows past M read as zeros
+    // A: pass i of a thread is row tid / CPR, chunk tid % CPR of the i-th slab of
+    // RPP rows; rows past M read as zeros
     const int arows = min(BM, M - m0);
-    const __amdgpu_buffer_rsrc_t a_r = __builtin_amdgcn_make_buffer_rsrc((void *)(aop + (size_t)m0 * K * EB), 0,
-                                                                         arows * K * EB, kRsrcWord3);
+    __amdgpu_buffer_rsrc_t a_r[ACH];
+#pragma unroll
+    for (int i = 0; i < ACH; i++) a_r[i] = row_slab(aop, m0 + RPP * i, RPP, M, K * EB);
     const __amdgpu_buffer_rsrc_t r_r =
         __builtin_amdgcn_make_buffer_rsrc((void *)(gsum + (size_t)m0 * G), 0, arows * G * 4, kRsrcWord3);
     const int ar0 = tid / CPR, ac = tid % CPR;
@@ -269,8 +271,7 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_mx_kernel(
     auto load_a = [&](int g, u32x4_t *ar, float &rs) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < ACH; i++)
-            ar[i] = __builtin_bit_cast(
-                u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(a_r, avo, (g * kGS + i * RPP * K) * EB, 0));
+            ar[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(a_r[i], avo, g * kGS * EB, 0));
         rs = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_r, rvo, g * 4, 0));
     };
     auto store_a = [&](int buf, const u32x4_t *ar, float rs) __attribute__((always_inline)) {

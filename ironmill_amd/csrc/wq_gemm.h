@@ -14,8 +14,9 @@
 // most ~7 vector instructions per MFMA (measured: 4 and 6 per MFMA are free,
 // 8 cost 1.4x; one wave per SIMD issues vector instructions at half that
 // rate).  So everything but the expansion and the fold is kept off the vector
-// unit: global addresses are a buffer resource per workgroup, one offset
-// register per thread and scalar stage offsets; LDS addresses are immediates.
+// unit: global addresses are buffer resources per workgroup (one per 16 rows of
+// the activation), one offset register per thread and a scalar offset along
+// the row; LDS addresses are immediates.
 //  * The weights go from memory straight into registers in the operand layout
 //    (lane = column + 32 x K half) and are expanded there: and-or places two
 //    codes beside the f16 exponent of 1024 (the upper nibble of a byte as 16 q,
@@ -95,6 +96,18 @@ __device__ __forceinline__ void tile_of(const TileOrder &o, int &mt, int &nt, in
     const int b = u / per_band, v = u - b * per_band;
     mt = b * o.band + v % o.band;
     nt = v / o.band;
+}
+
+// Rows [r0, r0 + n) of a row-major array of `rows` rows of `pitch` bytes as a
+// buffer of their own, the rows past the array left out of its size.  An access
+// whose vector offset holds row and column within the slab, and whose scalar
+// offset stays within a row, is in or out of bounds by its row alone -- also
+// where the bounds check leaves the scalar offset out, as it is specified to:
+// a row selected by the scalar offset would not be checked at all.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_slab(const void *base, int r0, int n, int rows, int pitch) {
+    const int first = min(r0, rows);
+    return __builtin_amdgcn_make_buffer_rsrc((void *)((const uint8_t *)base + (size_t)first * pitch), 0,
+                                             min(rows - first, n) * pitch, kRsrcWord3);
 }
 
 __device__ __forceinline__ uint32_t as_u32(half2_t h) { return __builtin_bit_cast(uint32_t, h); }
@@ -289,22 +302,23 @@ __global__ void __launch_bounds__(kThreads, 2) wq_gemm_kernel(const __half *__re
         }
     };
 
-    // A: chunk i of a thread is row 16 i + tid / 16, chunk tid % 16 of the group's
-    // rows (rows past M read as zeros); it lands in block (row / 32, k step cc & 7)
+    // A: chunk i of a thread is row tid / 16, chunk tid % 16 of the group's i-th
+    // slab of 16 rows (rows past M read as zeros); it lands in block (row / 32, k
+    // step cc & 7)
     const int arows = min(BM, M - m0);
     const __half *planes[2] = {a_hi, a_lo};
-    __amdgpu_buffer_rsrc_t a_r[NPL];
+    __amdgpu_buffer_rsrc_t a_r[NPL][ACH];
 #pragma unroll
     for (int p = 0; p < NPL; p++)
-        a_r[p] = __builtin_amdgcn_make_buffer_rsrc((void *)(planes[p] + (size_t)m0 * K), 0, arows * K * 2, kRsrcWord3);
+#pragma unroll
+        for (int i = 0; i < ACH; i++) a_r[p][i] = row_slab(planes[p], m0 + 16 * i, 16, M, K * 2);
     const int ar0 = tid >> 4, acc0 = tid & 15;
     const int avo = (ar0 * K + acc0 * 8) * 2;
     const int a_lds = (acc0 & 7) * kBlk + (ar0 + 32 * (acc0 >> 3)) * 16;
     auto load_a = [&](int g, int p, u32x4_t *ar) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < ACH; i++)
-            ar[i] = __builtin_bit_cast(u32x4_t,
-                                       __builtin_amdgcn_raw_buffer_load_b128(a_r[p], avo, (g * kGS + i * 16 * K) * 2, 0));
+            ar[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(a_r[p][i], avo, g * kGS * 2, 0));
     };
     auto store_a = [&](int buf, int p, const u32x4_t *ar) __attribute__((always_inline)) {
 #pragma unroll
@@ -577,7 +591,7 @@ __global__ void __launch_bounds__(kThreads, 2) wq_rows_kernel(const __half *__re
         }
     };
     // the activation: rows tid / 16 and + 16, chunk tid % 16 of each group (rows past M read as zeros)
-    const __amdgpu_buffer_rsrc_t x_r = __builtin_amdgcn_make_buffer_rsrc((void *)x, 0, M * K * 2, kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t x_r[2] = {row_slab(x, 0, 16, M, K * 2), row_slab(x, 16, 16, M, K * 2)};
     const __amdgpu_buffer_rsrc_t q_r =
         __builtin_amdgcn_make_buffer_rsrc((void *)(AWQ ? awq : x), 0, K * 2, kRsrcWord3);
     const int ar0 = tid >> 4, ac = tid & 15;
@@ -590,8 +604,8 @@ __global__ void __launch_bounds__(kThreads, 2) wq_rows_kernel(const __half *__re
         for (int i = 0; i < PB; i++) {
             const int g = min(g0 + i, g_end - 1);
             if (AWQ) qr[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(q_r, ac * 16, g * 256, 0));
-            xr[i][0] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_r, xvo, g * 256, 0));
-            if (two) xr[i][1] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_r, xvo, g * 256 + 32 * K, 0));
+            xr[i][0] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_r[0], xvo, g * 256, 0));
+            if (two) xr[i][1] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_r[1], xvo, g * 256, 0));
         }
     };
     constexpr int kSlot4[8] = {0, 4, 1, 5, 2, 6, 3, 7};

@@ -96,6 +96,29 @@ def test_library_exports_every_declared_symbol():
     assert sorted(_lib.SIGNATURES) == names  # the Python binding declares exactly these
 
 
+def test_buffer_loads_select_no_activation_row_by_scalar_offset():
+    """The scalar offset of a buffer load is left out of its bounds check, so it must not choose
+    the row of an array with fewer rows than a tile: no GEMM load's scalar offset holds a multiple
+    of K (the row pitch).  With one, the last tile of M = 17 or 65 rows read up to 48 rows past x."""
+    csrc = os.path.join(REPO, "ironmill_amd", "csrc")
+    loads = 0
+    for name in ("wq_gemm.h", "int4_gemm_mx.hip"):
+        text = open(os.path.join(csrc, name)).read()
+        for m in re.finditer(r"raw_buffer_load_b\d+\(", text):
+            args, depth, start, i = [], 0, m.end(), m.end()
+            while depth >= 0:   # split the call's arguments at the top level
+                c = text[i]
+                depth += (c in "([") - (c in ")]")
+                if depth < 0 or (c == "," and depth == 0):
+                    args.append(text[start:i])
+                    start = i + 1
+                i += 1
+            assert len(args) == 4, text[m.start():i]
+            assert not re.search(r"\bK\b", args[2]), f"{name}: scalar offset{args[2]} steps over rows"
+            loads += 1
+    assert loads >= 16
+
+
 def test_error_paths_without_gpu():
     L = _lib.lib
     assert L.imh_tq_cache_sizes(1, 8, 128, 64, None, None) == _lib.IMH_EINVAL
