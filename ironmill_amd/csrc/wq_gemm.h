@@ -4,8 +4,9 @@
 //     C[m][n] = f16( sum_g s[n][g] * sum_{k in g} a[m][k] * (q[n][k] - z[n][g]) ),  f32 accumulate
 //
 // a = x, or x / awq carried as f16 hi + lo planes (~22 bits, two products).
-// The weights are never rounded: INT4 codes enter as q - z (exact in f16 for
-// the integer zero-points of the quantizer), INT8 codes as f16 denormals
+// The weights are never rounded: INT4 codes enter as q - zi, zi the whole number
+// next to the zero-point (exact in f16), with what is left of a fractional or
+// very large zero-point applied in f32 to the group's sums; INT8 codes as f16 denormals
 // (q * 2^-24, exact) with the zero-point applied in f32 to the group's sums.
 //
 // What bounds it: the matrix cores (32 x 32 x 16: 32 cycles) against the
@@ -125,23 +126,49 @@ __device__ __forceinline__ float gate_act(float g, float u, int epi) {
     return act * u;
 }
 
-// The pair of f16 biases of an INT4 group: -(1024 + z) against 1024 + q, and
-// the same zero-point as rounded there, -(64 + z), against (1024 + 16 q) / 16.
-__device__ __forceinline__ uint32_t int4_bias(uint16_t zbits) {
+// The column constants of a group.  INT8: (scale * 2^24, -zero) as f32.  INT4:
+// the scale as f32, and the zero-point z split into the whole number zi within
+// +-1024 next to it, which the code expansion subtracts (q - zi is exact in
+// f16), and the rest z - zi (exact in f16 for every z), which is 0 for the
+// quantizer's ordinary zero-points and otherwise folded in f32 against the rows'
+// sums: halves {-(1024 + zi), z - zi}.
+template <int BITS>
+__device__ __forceinline__ u32x2_t column_consts(uint16_t s, uint16_t zbits) {
     const _Float16 z = __builtin_bit_cast(_Float16, zbits);
-    const _Float16 b1 = (_Float16)(-(1024.0f + (float)z));
-    const _Float16 b16 = (_Float16)((float)b1 + 960.0f);
-    return as_u32((half2_t){b1, b16});
+    const float sf = (float)__builtin_bit_cast(_Float16, s);
+    if (BITS == 4) {
+        const _Float16 zi = __builtin_elementwise_roundeven(
+            __builtin_amdgcn_fmed3h(z, (_Float16)-1024.0f, (_Float16)1024.0f));
+        return (u32x2_t){__builtin_bit_cast(uint32_t, sf), as_u32((half2_t){(_Float16)-1024.0f - zi, z - zi})};
+    }
+    return (u32x2_t){__builtin_bit_cast(uint32_t, sf * kTwo24), __builtin_bit_cast(uint32_t, -(float)z)};
 }
 
-// the column constants of a group: INT4 (scale f32, bias pair); INT8 (scale *
-// 2^24, -zero) as f32
-template <int BITS>
-__device__ __forceinline__ u32x2_t column_consts(uint16_t s, uint16_t z) {
-    const float sf = (float)__builtin_bit_cast(_Float16, s);
-    if (BITS == 4) return (u32x2_t){__builtin_bit_cast(uint32_t, sf), int4_bias(z)};
-    return (u32x2_t){__builtin_bit_cast(uint32_t, sf * kTwo24),
-                     __builtin_bit_cast(uint32_t, -(float)__builtin_bit_cast(_Float16, z))};
+// INT4: the second word's bias against 1024 + q, and -(64 + zi) against (1024 + 16 q) / 16
+__device__ __forceinline__ uint32_t code_bias(uint32_t cz) { return __builtin_amdgcn_perm(cz, cz, 0x01000100u); }
+__device__ __forceinline__ uint32_t code_bias16(uint32_t b1) {
+    return as_u32(as_h2(b1) + (half2_t){(_Float16)960.0f, (_Float16)960.0f});
+}
+
+// Some column of the wave has a zero-point with a rest (c0, c1: second words).
+__device__ __forceinline__ bool any_zero_rest(uint32_t c0, uint32_t c1) {
+    return __builtin_amdgcn_ballot_w64((c0 | c1) >> 16) != 0;
+}
+
+// The sums of 32 rows of a group over its operand (NPL planes, `plane` bytes
+// apart), as the products see it, laid out as a result: products with ones.
+template <int NPL, int UNROLL>
+__device__ __forceinline__ float16_t row_sums(const uint8_t *ab, int plane) {
+    const uint32_t one = 0x3C003C00u;
+    const half8_t ones = __builtin_bit_cast(half8_t, (u32x4_t){one, one, one, one});
+    float16_t r = {};
+#pragma unroll UNROLL
+    for (int st = 0; st < 8; st++)
+#pragma unroll
+        for (int p = 0; p < NPL; p++)
+            r = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8_t *>(ab + p * plane + st * kBlk),
+                                                       ones, r, 0, 0, 0);
+    return r;
 }
 
 // One prep launch.  Workgroups below `ablocks`: the activation planes -- hi =
@@ -379,19 +406,19 @@ __global__ void __launch_bounds__(kThreads, 2) wq_gemm_kernel(const __half *__re
     // group's loads issued and its activation stored between them (hook), then
     // the fold.  cur[half] holds the group's codes, cc its column constants.
     auto compute = [&](int buf, BRegs *cur, const u32x2_t *cc, auto &&hook) __attribute__((always_inline)) {
-        float sc[2];
-        uint32_t b1[2] = {}, b16[2] = {};
-        float nz[2] = {};
+        float sc[2], nz[2] = {};
+        uint32_t cz[2], b1[2] = {}, b16[2] = {};
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const u32x2_t c = SZT ? cc[j] : column_consts<BITS>((uint16_t)cc[j][0], (uint16_t)cc[j][1]);
-            const uint32_t cs = c[0], cz = c[1];   // scalars: a bit cast of a vector element takes element 0
+            const uint32_t cs = c[0];   // scalars: a bit cast of a vector element takes element 0
+            cz[j] = c[1];
             sc[j] = __builtin_bit_cast(float, cs);
             if (BITS == 4) {
-                b1[j] = __builtin_amdgcn_perm(cz, cz, 0x01000100u);
-                b16[j] = __builtin_amdgcn_perm(cz, cz, 0x03020302u);
+                b1[j] = code_bias(cz[j]);
+                b16[j] = code_bias16(b1[j]);
             } else {
-                nz[j] = __builtin_bit_cast(float, cz);
+                nz[j] = __builtin_bit_cast(float, cz[j]);
             }
         }
         const uint8_t *ab = &As[buf][0][lane * 16];
@@ -430,6 +457,18 @@ __global__ void __launch_bounds__(kThreads, 2) wq_gemm_kernel(const __half *__re
                         gg[mi][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[st & 1][p][mi], bf[st & 1][j],
                                                                            st == 0 && p == 0 ? zero16 : gg[mi][j], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
+        }
+        if (BITS == 4 && any_zero_rest(cz[0], cz[1])) {
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++) {
+                const float16_t rs = row_sums<NPL, 8>(ab + mi * 8 * kBlk, PLANE);
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const float rest = (float)as_h2(cz[j])[1];
+#pragma unroll
+                    for (int i = 0; i < 16; i++) gg[mi][j][i] = __builtin_fmaf(-rest, rs[i], gg[mi][j][i]);
+                }
+            }
         }
 #pragma unroll
         for (int mi = 0; mi < MI; mi++) {
@@ -652,17 +691,19 @@ __global__ void __launch_bounds__(kThreads, 2) wq_rows_kernel(const __half *__re
     for (int j = 0; j < 2; j++)
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[j][i] = 0.0f;
+    uint32_t rests = 0;   // INT4: the high halves tell whether a column of the block has a zero-point with a rest
     auto compute = [&](int i) __attribute__((always_inline)) {
         float sc[2], nz[2];
-        uint32_t b1[2], b16[2];
+        uint32_t cz[2], b1[2], b16[2];
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const u32x2_t c = column_consts<BITS>(bs[i][j], bz[i][j]);
-            const uint32_t cs = c[0], cz = c[1];   // scalars: a bit cast of a vector element takes element 0
+            const uint32_t cs = c[0];   // scalars: a bit cast of a vector element takes element 0
+            cz[j] = c[1];
             sc[j] = __builtin_bit_cast(float, cs);
-            nz[j] = __builtin_bit_cast(float, cz);
-            b1[j] = __builtin_amdgcn_perm(cz, cz, 0x01000100u);
-            b16[j] = __builtin_amdgcn_perm(cz, cz, 0x03020302u);
+            nz[j] = __builtin_bit_cast(float, cz[j]);
+            b1[j] = code_bias(cz[j]);
+            b16[j] = code_bias16(b1[j]);
         }
         const float16_t zero16 = {};
         float16_t gg[2];
@@ -697,6 +738,7 @@ __global__ void __launch_bounds__(kThreads, 2) wq_rows_kernel(const __half *__re
                 for (int j = 0; j < 2; j++)
                     gg[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[p], bf[j], st == 0 && p == 0 ? zero16 : gg[j], 0, 0, 0);
         }
+        if (BITS == 4) rests |= cz[0] | cz[1];
         float4_t rs[4];
         if (BITS == 8) {
 #pragma unroll
@@ -727,6 +769,24 @@ __global__ void __launch_bounds__(kThreads, 2) wq_rows_kernel(const __half *__re
         for (int i = 0; i < PB; i++) {
             if (g0 + i < g_end) compute(i);
             if (more) load_b(i, min(g0 + PB + i, g_end - 1));
+        }
+        // one branch per block (one per group: 2 % of the launch), the constants read once more
+        if (BITS == 4 && any_zero_rest(rests, 0)) {
+#pragma unroll 1
+            for (int i = 0; i < min(PB, g_end - g0); i++) {
+                const float16_t rs = row_sums<NPL, 1>(&As[i][0][lane * 16], PLANE);
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const int so = (g0 + i) * 2;
+                    const u32x2_t c = column_consts<BITS>(__builtin_amdgcn_raw_buffer_load_b16(s_r[j], svo[j], so, 0),
+                                                          __builtin_amdgcn_raw_buffer_load_b16(z_r[j], svo[j], so, 0));
+                    const uint32_t cs = c[0], cz = c[1];
+                    const float f = __builtin_bit_cast(float, cs) * (float)as_h2(cz)[1];
+#pragma unroll
+                    for (int k = 0; k < 16; k++) acc[j][k] = __builtin_fmaf(-f, rs[k], acc[j][k]);
+                }
+            }
+            rests = 0;
         }
         if (more) __syncthreads();   // the planes are rewritten next
     }

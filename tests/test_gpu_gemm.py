@@ -250,6 +250,55 @@ def test_gemm_rows_gate_up(dev, stream, act):
     assert np.all(err <= bound), f"worst {np.max(err / bound):.2f} of the bound"
 
 
+# zero-points as any f16 array may hold them: halves and smaller fractions, negative ones,
+# odd whole numbers past 1024 and past 2048, and far ones (not so far that y passes the f16 range)
+ZEROS = [7.5, 3.25, 0.1, -3.5, -1000.5, 1025.0, 1501.0, 2001.0, -1501.0, 3002.0, -5004.0, 8008.0, 8.0, 0.0]
+
+
+def any_zeros(q, seed):
+    """q with zero-points of ZEROS; every third column keeps its own, whole and small."""
+    z = np.random.default_rng(seed).choice(np.asarray(ZEROS, np.float16), q.zeros.shape)
+    z[::3] = q.zeros[::3]
+    q.zeros = z
+    return q
+
+
+def magnitudes(q):
+    """(|q| + |z|) s per weight: what sums of codes and of zero-points carry apart."""
+    codes = np.empty((q.n, q.k), np.float64)
+    codes[:, 0::2], codes[:, 1::2] = q.data & 0xF, q.data >> 4
+    return (codes + np.repeat(np.abs(q.zeros.astype(np.float64)), q.group_size, axis=1)) \
+        * np.repeat(q.scales.astype(np.float64), q.group_size, axis=1)
+
+
+@pytest.mark.parametrize("awq", [False, True])
+@pytest.mark.parametrize("m", [8, 9, 12, 17, 31, 32, 40, 65])
+def test_any_zero_points(dev, stream, m, awq):
+    """y = x . ((q - z) s) for every f16 z, on the matvec (8 rows), the one-launch kernel (9 to
+    32) and the tiles above it, one matrix and a pair: 2 f16 steps plus 2^-16 of the magnitudes
+    that sums of codes and zero-points carry (f32 sums; the activation's 22 bits against codes,
+    in the matvec up to 16 times the code).  A zero-point half a code off is past the bound in
+    the columns without a far one."""
+    n, k = 12801, 1152
+    w, s = weight(n, k, 17, awq)
+    q0 = any_zeros(quant.quantize_int4(w, awq_scales=s), 18)
+    q1 = any_zeros(quant.quantize_int4(weight(n, k, 19, False)[0], awq_scales=s), 20)
+    x16 = acts(m, k, m)
+    xd = dev.upload(x16)
+    w0, w1 = ops.AffineQuantizedWeight(dev, q0), ops.AffineQuantizedWeight(dev, q1)
+    y, g, u = (dev.empty((m, n), np.float16) for _ in range(3))
+    ops.encode_projection(stream, xd, w0, y, m)
+    ops.encode_batched_affine_matvec_int4(stream, xd, w0, g, w1, u, m)
+    stream.sync()
+    a = x16.astype(np.float64) if s is None else x16.astype(np.float64) / s.astype(np.float16).astype(np.float64)
+    for what, got, q in (("one matrix", y, q0), ("gate", g, q0), ("up", u, q1)):
+        exact = a @ exact_weights(q).T
+        bound = 2.0 * np.spacing(np.abs(exact).astype(np.float16)).astype(np.float64) \
+            + 2.0 ** -16 * (np.abs(a) @ magnitudes(q).T)
+        err = np.abs(got.read().astype(np.float64) - exact)
+        assert np.all(err <= bound), f"{what}: worst {np.max(err / bound):.2f} of the bound"
+
+
 def test_gemm_capture_reads_constants_in_place(dev):
     """Under capture with scratch for the activation planes only, the GEMM reads scales and
     zero-points in place: the replays equal the eager result bit for bit."""
