@@ -23,8 +23,8 @@
 //    (subnormals and the first binade), the matrix core's block scale 2^9
 //    restores q, and the correction subtracts z sum a.  The correction is one more
 //    matrix-core product per tile and group (the row sum split into three
-//    exact bf16 pieces against -c; the last of the group's bf16 products),
-//    so the fold of a group is one multiply-add.
+//    exact bf16 pieces, against -128 and -z as two; the last of the group's bf16
+//    products), so the fold of a group is one multiply-add.
 //  * a prep kernel writes the operand rows (x / awq rounded, each 8-element
 //    chunk in the slot order the code unpack produces) and their group sums.
 //    (INT4 codes beside a bf16 exponent: one and-or per two codes.)
@@ -78,13 +78,14 @@ enum Prec : int { PREC_BF16 = 1, PREC_FP8 = 2 };
 constexpr uint32_t kScaleCodesE8m0 = 0x88888888u;
 constexpr uint32_t kScaleOneE8m0 = 0x7F7F7F7Fu;
 
-// the column constants of a group: scale f32, and the correction's factor -c
-// (c = 128 + z for the bf16 codes, which carry 128; z for fp8) as a bf16 pair
-template <int P>
+// the column constants of a group: scale f32, and -z as two bf16 halves whose
+// sum it is exactly (an f16 has 11 significant bits, a bf16 8)
 __device__ __forceinline__ u32x2_t mx_consts(uint16_t s, uint16_t z) {
-    const __bf16 c = (__bf16)((P == PREC_BF16 ? -128.0f : 0.0f) - (float)__builtin_bit_cast(_Float16, z));
-    const uint32_t cb = __builtin_bit_cast(uint16_t, c);
-    return (u32x2_t){__builtin_bit_cast(uint32_t, (float)__builtin_bit_cast(_Float16, s)), cb | (cb << 16)};
+    const float nz = -(float)__builtin_bit_cast(_Float16, z);
+    const __bf16 c0 = (__bf16)nz;
+    const __bf16 c1 = (__bf16)(nz - (float)c0);
+    return (u32x2_t){__builtin_bit_cast(uint32_t, (float)__builtin_bit_cast(_Float16, s)),
+                     (uint32_t)__builtin_bit_cast(uint16_t, c0) | (uint32_t)__builtin_bit_cast(uint16_t, c1) << 16};
 }
 
 // Workgroups below ablocks: chunk c (8 elements) of the rows: a = x / awq (no
@@ -115,7 +116,7 @@ __global__ void __launch_bounds__(256) gemm_mx_prep_kernel(const __bf16 *__restr
         }
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            if (g0 + i < G) szt[(size_t)(g0 + i) * N + n] = mx_consts<P>(sv[i], zv[i]);
+            if (g0 + i < G) szt[(size_t)(g0 + i) * N + n] = mx_consts(sv[i], zv[i]);
         return;
     }
     const size_t cr = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -285,9 +286,9 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_mx_kernel(
         const float e1 = rs - (float)r0;
         const __bf16 r1 = (__bf16)e1;
         const __bf16 r2 = (__bf16)(e1 - (float)r1);
+        auto bits = [](__bf16 v) { return (uint32_t)__builtin_bit_cast(uint16_t, v); };
         Cs[buf][tid & (BM - 1)] =
-            (u32x4_t){(uint32_t)__builtin_bit_cast(uint16_t, r0) | ((uint32_t)__builtin_bit_cast(uint16_t, r1) << 16),
-                      (uint32_t)__builtin_bit_cast(uint16_t, r2), 0u, 0u};
+            (u32x4_t){bits(r0) | bits(r1) << 16, bits(r2) | bits(r0) << 16, bits(r1) | bits(r2) << 16, 0u};
     };
 
     float16_t acc[MI][2];
@@ -304,19 +305,26 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_mx_kernel(
     asm("v_mov_b32 %0, 0x43004300" : "=v"(exp128));
 
     // One group from LDS buffer buf: the MFMAs of the tiles over the group's k
-    // steps (hook(st): the next group's loads at k step st), the zero-point
-    // correction -c * rowsum as one more product (A lane (m, h): the row sum's
-    // three pieces, B lane (n, 0): -c three times, exact in bf16, lane (n, 1):
-    // zeros), then the fold with the scale of the lane's column.
+    // steps (hook(st): the next group's loads at k step st), the correction -(128
+    // + z) rowsum (fp8: -z rowsum) as one more product of exact bf16 pieces (A lane
+    // (m, h): the row sum's three pieces twice, B lane (n, 0): -128 (fp8: 0) three
+    // times, then the first half of -z, lane (n, 1): its second half three times,
+    // then zeros), then the fold with the scale of the lane's column.
+    constexpr uint32_t kOffset = P == PREC_BF16 ? 0xC300C300u : 0u;   // -128 twice
+    // byte selectors of B's words from the halves of -z (bytes 4-7) and kOffset (0-3)
+    const uint32_t cs0 = h ? 0x07060706u : 0x03020100u, cs1 = h ? 0x0C0C0706u : 0x05040100u,
+                   cs2 = h ? 0x0C0C0C0Cu : 0x05040504u;
     auto compute = [&](int buf, const BRegs &b, const u32x2_t *cc, auto &&hook) __attribute__((always_inline)) {
         float sc[2];
         bf16x8_t cb[2];
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const u32x2_t c = SZT ? cc[j] : mx_consts<P>((uint16_t)cc[j][0], (uint16_t)cc[j][1]);
-            const uint32_t cs = c[0], cz = h ? 0u : c[1];   // scalars: a bit cast of a vector element takes element 0
+            const u32x2_t c = SZT ? cc[j] : mx_consts((uint16_t)cc[j][0], (uint16_t)cc[j][1]);
+            const uint32_t cs = c[0], cz = c[1];   // scalars: a bit cast of a vector element takes element 0
             sc[j] = __builtin_bit_cast(float, cs);
-            cb[j] = __builtin_bit_cast(bf16x8_t, (u32x4_t){cz, cz & 0xFFFFu, 0u, 0u});
+            cb[j] = __builtin_bit_cast(bf16x8_t, (u32x4_t){__builtin_amdgcn_perm(cz, kOffset, cs0),
+                                                           __builtin_amdgcn_perm(cz, kOffset, cs1),
+                                                           __builtin_amdgcn_perm(cz, kOffset, cs2), 0u});
         }
         const uint8_t *ab = &As[buf][lane * 16];
         bf16x8_t ca[MI];

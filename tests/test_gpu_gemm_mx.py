@@ -109,6 +109,18 @@ def test_gemm_mx_tile_edges(dev, stream, prec, m, n, k, awq):
 
 
 @pytest.mark.parametrize("prec", [ops.GEMM_BF16, ops.GEMM_FP8_E4M3], ids=["bf16", "fp8"])
+@pytest.mark.parametrize("m,awq", [(1, False), (32, True), (65, True)])
+def test_gemm_mx_any_zero_points(dev, stream, prec, m, awq):
+    """Any f16 zero-point is exact, to the bound of whole and small ones: halves and smaller
+    fractions, negative ones, whole numbers that bf16 does not hold, and far ones."""
+    q, xb = problem(m, 513, 1152, 29 * m, awq)
+    z = np.asarray([7.5, 3.25, 0.1, -3.5, -1000.5, 129.0, 1025.0, 1501.0, -1501.0, 3002.0, 30000.0, 8.0], np.float16)
+    q.zeros = np.random.default_rng(m).choice(z, q.zeros.shape)
+    q.zeros[::3] = z[np.arange(q.zeros.shape[1]) % 4]   # a third of the columns near 0 throughout
+    check_exact(run(dev, stream, q, xb, prec), operand(xb, q, prec), q, f"m={m} awq={awq}")
+
+
+@pytest.mark.parametrize("prec", [ops.GEMM_BF16, ops.GEMM_FP8_E4M3], ids=["bf16", "fp8"])
 def test_gemm_mx_capture_reads_constants_in_place(dev, prec):
     """Under capture with scratch for the operand rows only, scales and zero-points are read
     in place: the replays equal the eager result bit for bit."""
