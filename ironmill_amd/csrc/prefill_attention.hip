@@ -66,6 +66,63 @@ __device__ __forceinline__ uint32_t tab_read(const uint8_t *tabs, uint32_t w, in
     return *reinterpret_cast<const uint32_t *>(tabs + off);
 }
 
+// One row of the FP16 kernel by a wave, in f32 over the row's own positions
+// [p_begin, lim) only (lane = position for the scores, two dims for the values):
+// what a row is given whose matrix-core result is not finite.  There a weight of
+// 0 (a position that the row does not see, or the low half of a weight) times an
+// infinite value of another row's position is NaN.
+__device__ __forceinline__ void exact_row(const imh::PrefillAttention &a, size_t head_base, size_t qrow,
+                                                    int p_begin, int lim, int S, int split) {
+    const int lane = threadIdx.x & 63;
+    const _Float16 *q = a.q + qrow * kD;
+    const _Float16 *k = reinterpret_cast<const _Float16 *>(a.k) + head_base * kD;
+    const _Float16 *v = reinterpret_cast<const _Float16 *>(a.v) + head_base * kD;
+    const float sl2 = a.attn_scale * 1.44269504f;
+    float m = -INFINITY, l = 0.0f, o0 = 0.0f, o1 = 0.0f;
+    for (int p0 = p_begin; p0 < lim; p0 += 64) {
+        float s = -INFINITY;
+        if (p0 + lane < lim) {
+            s = 0.0f;
+            for (int d = 0; d < kD; d += 8) {
+                const half8_t kv = *reinterpret_cast<const half8_t *>(k + (size_t)(p0 + lane) * kD + d);
+                for (int e = 0; e < 8; e++) s = __builtin_fmaf((float)q[d + e], (float)kv[e], s);
+            }
+            s *= sl2;
+        }
+        float nm = s;
+        for (int st = 32; st >= 1; st >>= 1) nm = fmaxf(nm, __shfl_xor(nm, st));
+        nm = fmaxf(nm, m);
+        const bool live = nm != -INFINITY;   // a row with no position yet keeps weight 0
+        const float corr = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - nm);
+        const float w = live && p0 + lane < lim ? __builtin_amdgcn_exp2f(s - nm) : 0.0f;
+        m = nm;
+        l = __builtin_fmaf(l, corr, w);
+        o0 *= corr;
+        o1 *= corr;
+        for (int j = 0; j < min(64, lim - p0); j++) {
+            const float wj = __shfl(w, j);
+            const half2_t vv = *reinterpret_cast<const half2_t *>(v + (size_t)(p0 + j) * kD + 2 * lane);
+            o0 = __builtin_fmaf(wj, (float)vv[0], o0);
+            o1 = __builtin_fmaf(wj, (float)vv[1], o1);
+        }
+    }
+    for (int st = 32; st >= 1; st >>= 1) l += __shfl_xor(l, st);
+    if (m == -INFINITY) o0 = o1 = 0.0f;
+    if (S > 1) {
+        const size_t pi = qrow * S + split;
+        a.part_o[pi * kD + 2 * lane] = o0;
+        a.part_o[pi * kD + 2 * lane + 1] = o1;
+        if (lane == 0) {
+            a.part_m[pi] = m;
+            a.part_l[pi] = l;
+        }
+    } else {
+        const float inv = 1.0f / fmaxf(l, 1e-10f);
+        a.out[qrow * kD + 2 * lane] = __float2half(o0 * inv);
+        a.out[qrow * kD + 2 * lane + 1] = __float2half(o1 * inv);
+    }
+}
+
 // grid (splits, kv heads, batch x row tiles), block 256 (TurboQuant 512).
 template <bool TQ>
 __global__ void __launch_bounds__(TQ ? 512 : 256) __attribute__((amdgpu_waves_per_eu(2, 2))) prefill_attention_kernel(
@@ -317,7 +374,8 @@ __global__ void __launch_bounds__(TQ ? 512 : 256) __attribute__((amdgpu_waves_pe
                 for (int i = 0; i < 16; i++) s[n][i] *= sl2;
         }
         // result i of block n is position p0 + 32 n + 8 (i >> 2) + 4 h + (i & 3)
-        if (p0 + kTile > lim_lo || p0 + kTile > p_end) {
+        const bool edge = p0 + kTile > lim_lo || p0 + kTile > p_end;   // of the positions some row sees
+        if (edge) {
 #pragma unroll
             for (int n = 0; n < NB; n++)
 #pragma unroll
@@ -358,6 +416,11 @@ __global__ void __launch_bounds__(TQ ? 512 : 256) __attribute__((amdgpu_waves_pe
                 const float4_t vs = *reinterpret_cast<const float4_t *>(&scl[TQ ? buf : 0][2][8 * q + 4 * h]);
 #pragma unroll
                 for (int j = 0; j < 4; j++) ph[q >> 1][4 * (q & 1) + j] = (_Float16)(s[0][4 * q + j] * vs[j]);
+            }
+            if (edge) {   // no weight where the row does not see the position, whatever its V scale
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    if (p0 + 8 * (i >> 2) + 4 * h + (i & 3) >= lim) ph[i >> 3][i & 7] = (_Float16)0.0f;
             }
             // operand i: step i / 8, V hi (i & 4 == 0) or lo, dim block i & 3
             auto read_v = [&](int i) __attribute__((always_inline)) {
@@ -441,7 +504,23 @@ __global__ void __launch_bounds__(TQ ? 512 : 256) __attribute__((amdgpu_waves_pe
         __syncthreads();
     }
     l_run += __shfl_xor(l_run, 32);
-    if (!row_ok) return;   // both lanes of a pair; no barrier follows
+    bool done = !row_ok;
+    if constexpr (!TQ) {
+        float any = 0.0f;   // NaN if a result is not finite
+#pragma unroll
+        for (int db = 0; db < 4; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) any = __builtin_fmaf(o[db][i], 0.0f, any);
+        const uint64_t lanes = __builtin_amdgcn_ballot_w64(row_ok && any != any);
+        const uint32_t again = (uint32_t)lanes | (uint32_t)(lanes >> 32);
+        for (uint32_t rest = again; rest; rest &= rest - 1) {
+            const int i = __builtin_ctz(rest), ri = w_first + i, ti = ri / a.gqa;
+            exact_row(a, head_base, ((size_t)b * a.T + ti) * a.nh + kvh * a.gqa + ri - ti * a.gqa, p_begin,
+                      min(L - a.T + ti + 1, p_end), S, split);
+        }
+        done = done || (again >> c & 1);
+    }
+    if (done) return;   // both lanes of a pair; no barrier follows
 
     // o[db][4 q + j]: dim 32 db + 8 q + 4 h + j of the lane's row
     if (S > 1) {   // the split's partial, maximum in log2 units (of the scale the weights have)

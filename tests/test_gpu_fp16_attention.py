@@ -191,3 +191,34 @@ def test_row_tile_kernel(dev, stream, nh, nkv, tokens, num_splits, lens, shift):
     ref = O.fp16_attention(q16, cache.k.read(), cache.v.read(), ctx, SCALE, nthreads=8,
                            seq_lens=np.asarray(lens, np.int32) if lens else None)
     assert_close(got, ref, what=f"row tiles T={tokens} nh={nh}")
+
+
+@pytest.mark.parametrize("nh,num_splits,aligned", [(32, 1, True), (16, 0, True), (8, 3, True), (8, 1, False)])
+def test_row_tile_non_finite_values(dev, stream, nh, num_splits, aligned):
+    """Infinite and NaN entries of K and V reach the tokens that see their position, as in the
+    oracle, and no earlier token of the chunk."""
+    batch, nkv, ctx, max_seq, tokens = 2, 8, 300, 320, 130
+    cache = fill_cache(dev, stream, batch, nkv, max_seq, ctx, seed=171)
+    k, v = cache.k.read(), cache.v.read()
+    v[0, 1, 297, 5] = np.inf     # seen by the last three tokens
+    v[0, 2, 200, 7] = -np.inf    # by a hundred, from token 30 on
+    v[0, 3, 10, 64] = np.inf     # by all
+    v[1, 0, 250, 100] = np.nan
+    k[1, 3, 299] = np.inf        # by the last token: its score is no number
+    cache.k.write(k)
+    cache.v.write(v)
+    q16 = np.random.default_rng(nh).standard_normal((batch, tokens, nh, D)).astype(np.float16)
+    shift = 0 if aligned else 2
+    qd, od = dev.buffer(q16.nbytes + 16), dev.buffer(q16.nbytes + 16)
+    qd.write(q16, shift)
+    ops.encode_fp16_attention(stream, cache, qd.ptr + shift, nh, ctx, od.ptr + shift, token_count=tokens,
+                              attn_scale=SCALE, num_splits=num_splits)
+    stream.sync()
+    got = od.read(np.float16, q16.shape, shift).astype(np.float32)
+    ref = O.fp16_attention(q16, k, v, ctx, SCALE, nthreads=8)
+    finite = np.isfinite(ref)
+    assert 0 < np.sum(~finite) < ref.size / 8
+    assert np.array_equal(np.isfinite(got), finite)
+    assert np.array_equal(np.isinf(got), np.isinf(ref))
+    assert np.array_equal(got[np.isinf(ref)] > 0, ref[np.isinf(ref)] > 0)
+    assert_close(got[finite], ref[finite], what=f"finite results, nh={nh}")

@@ -362,6 +362,29 @@ def test_attention_prefill_row_tiles(dev, stream, tq, tables, num_splits):
                 assert_close(got[bb, t], ref[bb], rel=5e-4, what=f"token {t} of seq {bb} (len {lt[bb]})")
 
 
+@pytest.mark.parametrize("num_splits", [1, 3])
+def test_row_tiles_infinite_value_scale(dev, stream, tq, tables, num_splits):
+    """An infinite V scale reaches the tokens that see its position and no earlier one."""
+    nkv, nh, batch, max_seq, tokens, ctx = 8, 16, 4, 1024, 129, 900
+    cache = fill_cache(dev, stream, tq, batch, nkv, max_seq, ctx, seed=95)
+    vs = cache.v_scales.read()
+    vs[1, 2, 880] = np.inf      # seen from token 109 on
+    cache.v_scales.write(vs)
+    q16 = np.random.default_rng(96).standard_normal((batch, tokens, nh, D)).astype(np.float16)
+    out = dev.empty((batch, tokens, nh, D), np.float16)
+    ops.encode_turboquant_attention(stream, tq, cache, dev.upload(q16), nh, ctx, out, 1.0 / math.sqrt(D),
+                                    num_splits=num_splits, token_count=tokens)
+    stream.sync()
+    got = out.read()
+    kc, vc, ks, _, kr = read_cache(cache)
+    for t in (0, 64, 95, 96, 108):
+        ref = O.tq_attention(q16[:, t], tables, kc, vc, ks, vs, kr, ctx - tokens + t + 1, 1.0 / math.sqrt(D), nthreads=8)
+        assert_close(got[:, t], ref, rel=5e-4, what=f"token {t}")
+    assert not np.isfinite(got[1, 109:, 4:6]).any()
+    got[1, 109:, 4:6] = 0
+    assert np.isfinite(got).all()
+
+
 def test_graph_replay_after_scratch_growth(dev, tq):
     """A graph keeps addressing the stream scratch it was captured with: a larger eager op
     that grows the scratch afterwards must not free it (the replay equals the eager run,
