@@ -413,14 +413,14 @@ int imh_encode_fp16_attention(imh_stream *stream, const imh_fp16_kv_cache *cache
     // 5 64 : 49, 16 109 : 51; GQA 1, T = 16 (32 blocks) 40 : 49 but at 2048
     // positions 19.6 : 18.6; 8 sequences at GQA 2, T = 2 103 : 102, 5 209 : 102
     const uint32_t blocks = B * nkv * qblocks;
-    if (token_count > 1 && !(blocks <= 16 || (blocks <= 32 && seq_len >= 8192)))
+    const uint32_t L = seq_lens && seq_len == 0 ? cache->max_seq_len : seq_len;   // the bound of the lengths
+    if (token_count > 1 && !(blocks <= 16 || (blocks <= 32 && L >= 8192)))
         return prefill_attention(stream, cache, q, num_heads, gqa, token_count, seq_len, seq_lens, attn_scale, out,
                                  num_splits);
 
     // KV split: ~512 workgroups, each split a multiple of one pass of the
     // workgroup's waves (64 positions); with per-sequence lengths the splits
-    // span the bound (0 = max_seq_len)
-    const uint32_t L = seq_lens && seq_len == 0 ? cache->max_seq_len : seq_len;
+    // span the bound
     uint32_t want = num_splits;
     if (want == 0) want = (512 + B * nkv * qblocks - 1) / (B * nkv * qblocks);
     const uint32_t max_splits = std::max<uint32_t>(1, (L + kSplitQuantum - 1) / kSplitQuantum);

@@ -222,3 +222,17 @@ def test_row_tile_non_finite_values(dev, stream, nh, num_splits, aligned):
     assert np.array_equal(np.isinf(got), np.isinf(ref))
     assert np.array_equal(got[np.isinf(ref)] > 0, ref[np.isinf(ref)] > 0)
     assert_close(got[finite], ref[finite], what=f"finite results, nh={nh}")
+
+
+@pytest.mark.parametrize("max_seq,tokens", [(8192, 16), (8191, 16), (8192, 17)])
+def test_bound_of_lengths_given_or_not(dev, stream, max_seq, tokens):
+    """seq_len 0 with seq_lens means max_seq_len, also for the choice of the kernel: the same
+    bits as with the bound written out, on both sides of the rule's lines."""
+    nkv, nh = 8, 8
+    cache = fill_cache(dev, stream, 1, nkv, max_seq, 400, seed=181)
+    q16 = np.random.default_rng(182).standard_normal((1, tokens, nh, D)).astype(np.float16)
+    got = [run_attention(dev, stream, cache, q16, nh, bound, seq_lens=[400]) for bound in (0, max_seq)]
+    assert np.array_equal(got[0].view(np.uint16), got[1].view(np.uint16))
+    ref = O.fp16_attention(q16, cache.k.read(), cache.v.read(), max_seq, SCALE, nthreads=8,
+                           seq_lens=np.asarray([400], np.int32))
+    assert_close(got[0], ref, what=f"T={tokens} bound {max_seq}")
