@@ -575,8 +575,17 @@ int imh_affine_gemm_int4(imh_stream *stream, const void *x, uint32_t M, const im
     order.tiles_n = (N + kCols - 1) / kCols;
     const int tiles = order.tiles_m * order.tiles_n;
     int splits = tiles < 2 * cus ? gemm_splits(tiles, G, (int)M, N, cus, P) : 1;
-    const int per = (G + splits - 1) / splits;
+    int per = (G + splits - 1) / splits;
     splits = (G + per - 1) / per;
+    // scratch slot 2: split partials; without room for them (a capture, or no
+    // memory) K is not split
+    void *part_scr = nullptr;
+    if (splits > 1 &&
+        !imh::stream_scratch_optional(stream, 2, (size_t)splits * M * N * sizeof(float), &part_scr)) {
+        splits = 1;
+        per = G;
+    }
+    float *part = splits > 1 ? static_cast<float *>(part_scr) : nullptr;
     order.splits = splits;
     // band: the largest divisor of tiles_m that is at most tiles_m / 8 (so
     // each XCD gets about one band), at least 1
@@ -588,7 +597,7 @@ int imh_affine_gemm_int4(imh_stream *stream, const void *x, uint32_t M, const im
         }
     // scratch slot 0: operand rows, group sums and, where it has room, the
     // transposed column constants (a stream capturing with the scratch of the
-    // first two reads scales and zero-points in place); slot 2: split partials
+    // first two reads scales and zero-points in place)
     const size_t a_bytes = ((size_t)M * K * eb + 255) / 256 * 256;
     const size_t gsum_bytes = ((size_t)M * G * sizeof(float) + 255) / 256 * 256;
     const size_t szt_bytes = (size_t)G * N * sizeof(u32x2_t);
@@ -602,13 +611,6 @@ int imh_affine_gemm_int4(imh_stream *stream, const void *x, uint32_t M, const im
     uint8_t *aop = static_cast<uint8_t *>(scr);
     float *gsum = reinterpret_cast<float *>(aop + a_bytes);
     u32x2_t *szt = reinterpret_cast<u32x2_t *>(aop + a_bytes + gsum_bytes);
-    float *part = nullptr;
-    if (splits > 1) {
-        void *p = nullptr;
-        rc = imh::stream_scratch(stream, 2, (size_t)splits * M * N * sizeof(float), &p);
-        if (rc) return rc;
-        part = static_cast<float *>(p);
-    }
     const __bf16 *xb = static_cast<const __bf16 *>(x);
     const __half *awq = reinterpret_cast<const __half *>(w->awq_scales);
     const size_t chunks = (size_t)M * K / 8;

@@ -314,15 +314,11 @@ int run_gemm(imh_stream *s, const ActIn &in, int M, const imh_affine_int4_weight
     const int cus = s->dev->props.multiProcessorCount;
     void *ws = nullptr;
     const size_t ws_bytes = gemm_workspace_bytes(M, N, K, nmat, cus);
-    int rc = IMH_OK;
-    // a capturing stream whose scratch lacks the partials runs the GEMM unsplit
-    if (ws_bytes && !(s->capturing && s->scratch_bytes[2] < ws_bytes)) {
-        rc = imh::stream_scratch(s, 2, ws_bytes, &ws);
-        if (rc) return rc;
-    }
+    // without room for the partials (a capture, or no memory) the GEMM runs unsplit
+    if (ws_bytes && !imh::stream_scratch_optional(s, 2, ws_bytes, &ws)) ws = nullptr;
     const __half *x = in.a;
     if (in.b) {   // residual + RMSNorm rows, then the projection of the normed rows
-        rc = encode_resnorm_rows(s, in.a, in.b, in.gamma, in.eps, in.residual_out, in.normed_out, M, K);
+        const int rc = encode_resnorm_rows(s, in.a, in.b, in.gamma, in.eps, in.residual_out, in.normed_out, M, K);
         if (rc) return rc;
         x = in.normed_out;
     }
@@ -432,13 +428,14 @@ int run_matvec(imh_stream *s, ActIn in, uint32_t B, int nmat, int epi, int N, in
 // at 9-31 rows 8.5 against 10-12; 3001 x 4096 at 9 / 12 / 24 rows 12.6 / 14.3 /
 // 20.9 against 13.0 / 13.4 / 14.7; 2560 x 9728 at 9 / 16 / 31 rows 23 / 33 / 43
 // against 15.5 / 16.9 / 19.5.  Only where the operand is the f16 rows as given
-// (a residual-norm source whose rows are not rounded first stays), and not when
-// a capturing stream's scratch lacks the split's partials.
+// (a residual-norm source whose rows are not rounded first stays).  A capturing
+// stream whose scratch lacks the split's partials stays on the matvec if it has
+// the operand image's; with neither it records the GEMM, which unsplit needs none.
 bool rows_gemm_pays(const imh_stream *s, const ActIn &in, int B, const imh_affine_int4_weight *w, int nmat) {
     if (B < 9 || (in.b && in.round_mode != 1)) return false;
     if ((double)B * w->n * w->k * nmat < 115e6) return false;
     const size_t ws = gemm_workspace_bytes(B, (int)w->n, (int)w->k, nmat, s->dev->props.multiProcessorCount);
-    return !(s->capturing && s->scratch_bytes[2] < ws);
+    return !s->capturing || s->scratch_bytes[2] >= ws || s->scratch_bytes[0] < image_bytes((uint32_t)B, w->k);
 }
 
 // Validates the weights and runs the op: x (plain) or the residual-norm

@@ -343,3 +343,43 @@ def test_gemm_capture_without_partials(dev, m):
         g.launch()
         st.sync()
         assert np.all(np.abs(y.read().astype(np.float64) - exact) <= bound)
+
+
+def rows_splits(m, n, k, nmat=1, cus=256):
+    """The K split of the one-launch kernel, as its host code picks it."""
+    tiles, g = -(-n // (256 // nmat)), k // 128
+    cost = {}
+    for per in range(4, g + 4, 4):
+        sp = -(-g // per)
+        cost.setdefault(sp, -(-tiles * sp // (2 * cus)) * (4 + 1.05 * min(per, g))
+                        + (3 + sp * m * nmat * n * 8 / 4.5e6 if sp > 1 else 0))
+    return min(cost, key=cost.get)
+
+
+@pytest.mark.parametrize("warm", [None, "gemm", "matvec"])
+def test_gemm_rows_capture(dev, warm):
+    """A capture of 12 rows whose stream lacks the split's partials -- with no scratch at all, with
+    that of a smaller projection on the same kernel, or with the matvec's operand image -- records
+    what needs none; each replay is within 2 f16 steps plus the sum-order slack of the exact value."""
+    m, n, k = 12, 6144, 9728
+    assert rows_splits(m, n, k) * m * n * 4 > 2 ** 20   # more than the smallest scratch block
+    w, s = weight(n, k, 161, True)
+    q = quant.quantize_int4(w, awq_scales=s)
+    x16 = acts(m, k, 162)
+    st = dev.stream()
+    xd, y, wt = dev.upload(x16), dev.empty((m, n), np.float16), ops.AffineQuantizedWeight(dev, q)
+    if warm:
+        n0 = 1024 if warm == "gemm" else 64   # 64 x 9728 x 12 is the matvec's, 1024 x 9728 x 12 the GEMM's
+        assert rows_splits(m, 1024, k) * m * 1024 * 4 <= 2 ** 20
+        w0 = ops.AffineQuantizedWeight(dev, quant.quantize_int4(w[:n0].copy(), awq_scales=s))
+        ops.encode_projection(st, xd, w0, dev.empty((m, n0), np.float16), m)
+    g = st.capture(lambda: ops.encode_projection(st, xd, wt, y, m))
+    a, W = x16.astype(np.float64) / s.astype(np.float16).astype(np.float64), exact_weights(q)
+    exact = a @ W.T
+    # the matvec's sums hold codes and zero-points apart
+    bound = 2.0 * np.spacing(np.abs(exact).astype(np.float16)).astype(np.float64) + 2.0 ** -16 * (np.abs(a) @ magnitudes(q).T)
+    for _ in range(2):
+        st.zero(y)
+        g.launch()
+        st.sync()
+        assert np.all(np.abs(y.read().astype(np.float64) - exact) <= bound)

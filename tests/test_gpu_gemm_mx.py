@@ -143,6 +143,40 @@ def test_gemm_mx_capture_reads_constants_in_place(dev, prec):
         assert np.array_equal(yg.read(), want)
 
 
+@pytest.mark.parametrize("prec", [ops.GEMM_BF16, ops.GEMM_FP8_E4M3], ids=["bf16", "fp8"])
+@pytest.mark.parametrize("m", [17, 32])
+def test_gemm_mx_few_rows_capture(dev, prec, m):
+    """32-row tiles under capture.  With scratch for the operand rows and the split's partials,
+    scales and zero-points are read in place, and the replays equal the eager result bit for bit;
+    without the partials K is not split, within the bound."""
+    n, k = 10000, 2048
+    q, xb = problem(m, n, k, 13 * m, True)
+    q0, _ = problem(m, 256, k, 14, True)
+    qf, _ = problem(m, 2560, 9728, 15, False)
+    xd, x16 = dev.upload(xb), dev.upload(np.zeros((m, 9728), np.float16))
+    w, w0, wf = (ops.AffineQuantizedWeight(dev, v) for v in (q, q0, qf))
+    ye, yg, y0 = dev.empty((m, n), np.uint16), dev.empty((m, n), np.uint16), dev.empty((m, 2560), np.uint16)
+    eager = dev.stream()
+    ops.encode_affine_gemm_int4(eager, xd, m, w, ye, prec)
+    eager.sync()
+    want = ye.read()
+    check_exact(O.bf16_to_f32(want), operand(xb, q, prec), q, f"eager m={m}")
+    for partials in (True, False):
+        st = dev.stream()
+        if partials:   # the f16 GEMM's partials fill slot 2 and leave slot 0 alone
+            ops.encode_projection(st, x16, wf, y0, m)
+        ops.encode_affine_gemm_int4(st, xd, m, w0, y0, prec)
+        g = st.capture(lambda: ops.encode_affine_gemm_int4(st, xd, m, w, yg, prec))
+        for _ in range(2):
+            st.zero(yg)
+            g.launch()
+            st.sync()
+            if partials:
+                assert np.array_equal(yg.read(), want)
+            else:
+                check_exact(O.bf16_to_f32(yg.read()), operand(xb, q, prec), q, f"unsplit m={m}")
+
+
 @pytest.mark.parametrize("m,n,k", [(512, 9728, 2560), (512, 2560, 9728), (2048, 9728, 2560), (2048, 2560, 9728)])
 def test_gemm_mx_configs3(dev, stream, m, n, k):
     """BASELINE configs[3] at its full sizes: X bf16 N(0,1), W INT4 g128 from N(0,0.02), bf16
