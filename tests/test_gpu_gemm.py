@@ -383,3 +383,38 @@ def test_gemm_rows_capture(dev, warm):
         g.launch()
         st.sync()
         assert np.all(np.abs(y.read().astype(np.float64) - exact) <= bound)
+
+
+def test_gemm_pair_capture_reads_constants_in_place(dev):
+    """Gate and up with AWQ under capture, with scratch for the activation planes only: both
+    matrices' scales and zero-points are read in place, and the replays equal the eager result bit
+    for bit."""
+    m, k = 1023, 2048
+    ws, s = weight(256, k, 191, True)
+    small = ops.AffineQuantizedWeight(dev, quant.quantize_int4(ws, awq_scales=s))
+    gate, up = (ops.AffineQuantizedWeight(dev, quant.quantize_int4(weight(8200, k, seed, False)[0], awq_scales=s))
+                for seed in (192, 193))
+    x16 = acts(m, k, 194)
+    st = dev.stream()
+    xd, y0 = dev.upload(x16), dev.empty((m, 256), np.float16)
+    outs = [dev.empty((m, 8200), np.float16) for _ in range(5)]
+
+    def run(act, g, u):
+        ops.encode_fused_ffn_gate_up_act_int4(st, xd, gate, up, act, m)
+        ops.encode_batched_affine_matvec_int4(st, xd, gate, g, up, u, m)
+    ops.encode_projection(st, xd, small, y0, m)
+    graph = st.capture(lambda: run(*outs[:3]))
+    st2 = dev.stream()
+    ops.encode_fused_ffn_gate_up_act_int4(st2, xd, gate, up, outs[3], m)
+    st2.sync()
+    want_act = outs[3].read().view(np.uint16)
+    ops.encode_batched_affine_matvec_int4(st2, xd, gate, outs[3], up, outs[4], m)
+    st2.sync()
+    want = [want_act, outs[3].read().view(np.uint16), outs[4].read().view(np.uint16)]
+    for _ in range(2):
+        for o in outs[:3]:
+            st.zero(o)
+        graph.launch()
+        st.sync()
+        for o, w in zip(outs, want):
+            assert np.array_equal(o.read().view(np.uint16), w)

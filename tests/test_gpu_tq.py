@@ -362,6 +362,38 @@ def test_attention_prefill_row_tiles(dev, stream, tq, tables, num_splits):
                 assert_close(got[bb, t], ref[bb], rel=5e-4, what=f"token {t} of seq {bb} (len {lt[bb]})")
 
 
+@pytest.mark.parametrize("num_splits", [0, 1, 3])
+@pytest.mark.parametrize("nh,tokens,lens", [
+    (32, 257, [900, 140, 300]),                 # GQA 4: four rows into a fifth tile; 120 tiles, 19.0 M pairs at the bound
+    (32, 65, [900, 900, 30, 65]),               # its four rows into a second tile; 64 tiles, 7.2 M pairs
+    (8, 257, [900, 256, 900, 900]),             # GQA 1: one row into a second tile; 64 tiles, 6.3 M pairs
+])
+def test_attention_prefill_row_tiles_gqa(dev, stream, tq, tables, nh, tokens, lens, num_splits):
+    """The row-tile kernel at the other head groups: rows map to (token, head) by them, and the
+    limits of a wave's 32 rows, the tail of the last tile included."""
+    nkv, batch, max_seq = 8, len(lens), 900
+    rows, bound = tokens * nh // nkv, max_seq
+    assert batch * nkv * -(-rows // 256) >= 32 and batch * nh * tokens * (bound - tokens // 2) >= 6e6 and rows % 256
+    cache = fill_cache(dev, stream, tq, batch, nkv, max_seq, 900, seed=97)
+    q16 = np.random.default_rng(98).standard_normal((batch, tokens, nh, D)).astype(np.float16)
+    out = dev.empty((batch, tokens, nh, D), np.float16)
+    lens = np.array(lens, np.int32)
+    ops.encode_turboquant_attention(stream, tq, cache, dev.upload(q16), nh, 0, out, 1.0 / math.sqrt(D),
+                                    seq_lens=dev.upload(lens), num_splits=num_splits, token_count=tokens)
+    stream.sync()
+    got = out.read()
+    kc, vc, ks, vs, kr = read_cache(cache)
+    for t in sorted({0, 1, 7, 8, 31, 32, 63, 64, tokens - 35, tokens - 2, tokens - 1}):
+        lt = np.maximum(lens - tokens + t + 1, 0).astype(np.int32)
+        ref = O.tq_attention(q16[:, t], tables, kc, vc, ks, vs, kr, max_seq, 1.0 / math.sqrt(D),
+                             seq_lens=lt, nthreads=8)
+        for bb in range(batch):
+            if lt[bb] == 0:
+                assert not got[bb, t].astype(np.float32).any()
+            else:
+                assert_close(got[bb, t], ref[bb], rel=5e-4, what=f"token {t} of seq {bb} (len {lt[bb]})")
+
+
 @pytest.mark.parametrize("num_splits", [1, 3])
 def test_row_tiles_infinite_value_scale(dev, stream, tq, tables, num_splits):
     """An infinite V scale reaches the tokens that see its position and no earlier one."""
