@@ -414,7 +414,8 @@ int imh_encode_fp16_attention(imh_stream *stream, const imh_fp16_kv_cache *cache
     // positions 19.6 : 18.6; 8 sequences at GQA 2, T = 2 103 : 102, 5 209 : 102
     const uint32_t blocks = B * nkv * qblocks;
     const uint32_t L = seq_lens && seq_len == 0 ? cache->max_seq_len : seq_len;   // the bound of the lengths
-    if (token_count > 1 && !(blocks <= 16 || (blocks <= 32 && L >= 8192)))
+    // The row tiles address a head's rows by 32-bit byte offsets: longer caches stay here.
+    if (token_count > 1 && L <= 0x7FFFFF && !(blocks <= 16 || (blocks <= 32 && L >= 8192)))
         return prefill_attention(stream, cache, q, num_heads, gqa, token_count, seq_len, seq_lens, attn_scale, out,
                                  num_splits);
 

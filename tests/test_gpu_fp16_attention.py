@@ -236,3 +236,19 @@ def test_bound_of_lengths_given_or_not(dev, stream, max_seq, tokens):
     ref = O.fp16_attention(q16, cache.k.read(), cache.v.read(), max_seq, SCALE, nthreads=8,
                            seq_lens=np.asarray([400], np.int32))
     assert_close(got[0], ref, what=f"T={tokens} bound {max_seq}")
+
+
+def test_chunk_over_a_cache_past_32_bit_offsets(dev, stream):
+    """A head of more than 2^24 positions, 4 GiB each of K and V: a chunk reads the rows past
+    that.  K is 0, so every visible position weighs the same; V is 0 but for the last 4096."""
+    tokens, ctx, ones = 160, 2 ** 24 + 4096, 4096
+    cache = ops.Fp16KvCache(dev, 1, 1, D, ctx)
+    cache.zero(stream)
+    stream.sync()
+    cache.v.write(np.full((ones, D), 16384.0, np.float16), 2 * D * (ctx - ones))
+    q16 = np.random.default_rng(191).standard_normal((1, tokens, 1, D)).astype(np.float16)
+    got = run_attention(dev, stream, cache, q16, 1, ctx).astype(np.float64)
+    seen = ctx - tokens + 1 + np.arange(tokens)
+    exact = 16384.0 * (seen - (ctx - ones)) / seen
+    # f16 rounding of the result, 2^-11, and f32 sums of up to 2^17 equal terms per wave
+    assert np.all(np.abs(got - exact[None, :, None, None]) <= 2.0 ** -9 * exact[None, :, None, None])
