@@ -212,8 +212,9 @@ typedef struct {
 /* superblock_matvec_int8 (affine_matvec.metal:123-189) for token_count rows:
  * y[t][r] = f16( sum_k (x[t][k] / awq[k]) * (q[r][k] - z) * s ), f32 accumulate.
  * x [token_count][k] f16, y [token_count][n] f16.  From 9 rows (4 for large
- * weights) a GEMM over operand planes in the stream's scratch; a capture whose
- * stream lacks that scratch records the matvec, which needs none. */
+ * weights) a GEMM, which uses the stream's scratch for its split partials and,
+ * past 32 rows, its operand planes; a capture whose stream lacks that scratch
+ * records the matvec, which needs none. */
 int imh_encode_affine_projection_int8(imh_stream *stream, const uint16_t *x, uint32_t token_count,
                                       const imh_affine_int8_weight *w, uint16_t *y);
 

@@ -16,8 +16,8 @@ constexpr int kGemmMinTokens = 32;
 int gemm_splits(int M, int N, int K, int nmat, int cus);
 // bytes of f32 split partials encode_gemm uses (0 without a split)
 size_t gemm_workspace_bytes(int M, int N, int K, int nmat, int cus);
-// y0 [M][N] f16 = f16(x [M][K] / awq0) . W0^T with W0's dequantized f16
-// values; with w1 (a gate/up pair sharing x and awq0): epi 0 also stores
+// y0 [M][N] f16 = (x [M][K] / awq0) . W0^T, x / awq0 to ~22 bits and W0's
+// exact values (q - z) s; with w1 (a gate/up pair sharing x and awq0): epi 0 also stores
 // y1 = x . W1^T, epi 2 / 3 stores y0 = f16(silu / gelu(x . W0^T) * (x . W1^T))
 // from the f32 results.  workspace NULL: K is not split.
 int encode_gemm(imh_stream *s, const __half *x, int M, const imh_affine_int4_weight *w0,

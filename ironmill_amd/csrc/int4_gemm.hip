@@ -135,9 +135,10 @@ __global__ void __launch_bounds__(256) resnorm_rows_kernel(const __half *__restr
 
 namespace imh_int4 {
 
-// K splits of the one-launch kernel: a split takes whole blocks of groups; a
-// round of workgroups (two per CU) costs ~4 us and ~1.05 per group, a split
-// ~3 us of reduction and its partials' round trip.  Measured at 12 rows, AWQ,
+// K splits of the one-launch kernel, counted in whole blocks of groups (the
+// launch then balances the splits by groups: G = 9 at 3 splits gives 3 each, not
+// 4, 4 and 1); a round of workgroups (two per CU) costs ~4 us and ~1.05 per
+// group, a split ~3 us of reduction and its partials' round trip.  Measured at 12 rows, AWQ,
 // 9728 -> 2560: 1 / 2 / 3 / 5 blocks per split 16.1 / 18.9 / 20 / 33 us.
 int rows_splits(int M, int N, int K, int nmat, int cus) {
     const int tiles = (N + 256 / nmat - 1) / (256 / nmat), G = K / kGS;
@@ -158,9 +159,11 @@ int rows_splits(int M, int N, int K, int nmat, int cus) {
 
 // K splits (whole groups each, at least 4 per split), only as many as keep
 // the grid within one round of workgroup slots (two per CU).  Each
-// workgroup costs about the same per group (kGroupUs at two per CU, ~0.6 of
-// that alone on a CU), and a split adds its partials' round trip (read back
-// by the reduce launch at ~4.5 TB/s plus ~2 us).
+// workgroup is taken to cost the same per group (g2 = 2.2 us at two per CU, 0.6
+// of that alone on a CU; one value for one plane, two planes and INT8 -- traced,
+// two planes take 3.8-4.2 at two per CU, INT8 2.9 alone on its CU), and a split
+// adds its partials' round trip (read back by the reduce launch at ~4.5 TB/s plus
+// ~2 us).
 int gemm_splits(int M, int N, int K, int nmat, int cus) {
     if (M <= kRowsMax) return rows_splits(M, N, K, nmat, cus);
     const int bm = 64;

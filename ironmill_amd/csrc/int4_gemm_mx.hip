@@ -15,9 +15,8 @@
 //    weight column + 32 x K half, two 16-byte loads per lane per group and
 //    32-column fragment) and is expanded there, so a workgroup's weights
 //    never touch LDS and each is read once per workgroup.
-//  * bf16: a code byte q placed under the bf16 exponent byte 0x43 is the bf16
-//    value 128 + q exactly (one v_perm per two codes); the MFMA gives
-//    sum a (128 + q) and the group's correction subtracts (128 + z) sum a,
+//  * bf16: a code q beside the bf16 exponent byte 0x43 is the bf16 value 128 + q
+//    exactly (a shift and one and-or per two codes); the MFMA gives sum a (128 + q) and the group's correction subtracts (128 + z) sum a,
 //    with sum a the row's group sum of the rounded operand (exact products,
 //    f32 sums).  fp8: the code byte itself, read as e4m3, is q * 2^-9 exactly
 //    (subnormals and the first binade), the matrix core's block scale 2^9
@@ -27,7 +26,6 @@
 //    products), so the fold of a group is one multiply-add.
 //  * a prep kernel writes the operand rows (x / awq rounded, each 8-element
 //    chunk in the slot order the code unpack produces) and their group sums.
-//    (INT4 codes beside a bf16 exponent: one and-or per two codes.)
 //  * the 32 x 32 matrix-core shapes (v_mfma_f32_32x32x16_bf16,
 //    v_mfma_scale_f32_32x32x64_f8f6f4): measured on the MI355X they sustain
 //    ~2.3 / ~4.9 PFLOP/s where the 16 x 16 bf16 shape stops at ~1.7.
@@ -510,8 +508,10 @@ int check_gemm_weight(const imh_affine_int4_weight *w, const char *who) {
 
 // K splits for a grid of `tiles` output tiles (fewer than the slots, two
 // per CU).  Workgroups of a launch are dispatched as slots free up, and each
-// costs about the same per group: ~2.4 us bf16 / ~1.9 us fp8 with two per
-// CU, ~0.9 of that alone on its CU.  So a grid of W workgroups runs full
+// is taken to cost the same per group: 2.4 us bf16 / 1.9 us fp8 with two per
+// CU, 0.9 of that alone on its CU, and the same for 32-row tiles.  These were
+// fitted to the tiling before this one (traced now: 2.7 bf16, 2.5 fp8 for 64
+// rows), and not to the 32-row tiles.  So a grid of W workgroups runs full
 // rounds of two per CU, then its remainder (one per CU where it fits); a
 // split adds the partials' round trip (written during the GEMM, read back by
 // the reduce launch at ~4.5 TB/s plus ~2 us).  Measured against the earlier

@@ -28,7 +28,7 @@
 // Measured (us, write + attention, before -> after): FP16, two sequences of up
 // to 2500 positions, T = 301, 16 / 8 heads 242 -> 46; one of 8192, T = 512, 32
 // / 8 heads 1354 -> 126; TurboQuant at the latter sizes 403 -> 264.  The
-// TurboQuant kernel keeps the matrix cores busy 54 % of the time: its score
+// TurboQuant kernel keeps the matrix cores busy 53 % of the time: its score
 // sums are one chain of 40 dependent products per 32 positions, and the
 // registers (128 for the query planes, 64 for the result) leave no room for a
 // second chain.
@@ -745,8 +745,9 @@ int launch_prefill_combine(imh_stream *s, bool tq, size_t rows, uint32_t splits,
 
 // KV splits: the count (each at least 256 positions) that gives the fewest
 // rounds of workgroup slots -- two workgroups per CU for the FP16 kernel, one
-// for the TurboQuant kernel (LDS) -- per split, a split's partials costing
-// about 0.5 % of the unsplit round.
+// for the TurboQuant kernel (LDS) -- per split, a split costing a flat 0.5 % of
+// the unsplit round, whatever the bytes of its partials (520 per row, written
+// and read: 2 x 31 MB for the six splits of 9632 rows).
 uint32_t prefill_splits(bool tq, uint32_t groups, uint32_t L, int cus) {
     const uint32_t slots = (uint32_t)cus * (tq ? 1 : 2);
     uint32_t best = 1;

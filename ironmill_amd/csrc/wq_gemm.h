@@ -38,11 +38,11 @@
 //
 // Measured (us, before -> after; before: 128 x 128 tiles of 16 x 16 MFMAs with
 // both operands through LDS, and for INT8 the 8-row matvec once per 8 rows):
-// FFN block 2560 / 9728 with AWQ at 777 rows 467 -> 243 (of it gate + up 320 ->
-// 150, ~1000 TFLOP/s counting both planes), INT8 9728 -> 2560 at 200 rows 1184
-// -> 43.  The matrix cores are busy 70 % of a resident wave's time; freezing
-// the addresses of the activation and weight loads changes nothing, a quarter
-// of the fold saves 6 %.
+// FFN block 2560 / 9728 with AWQ at 777 rows 466 -> 245 (of it gate + up 320 ->
+// ~155, ~1000 TFLOP/s counting both planes), INT8 9728 -> 2560 at 200 rows 1180
+// -> 43.  The matrix cores are busy 71 % of the time that a SIMD has waves (gate +
+// up; no LDS bank conflicts); freezing the addresses of the activation and
+// weight loads changes nothing, a quarter of the fold saves 6 %.
 #pragma once
 
 #include <hip/hip_runtime.h>
