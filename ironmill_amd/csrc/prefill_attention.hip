@@ -72,7 +72,7 @@ __device__ __forceinline__ uint32_t tab_read(const uint8_t *tabs, uint32_t w, in
 // 0 (a position that the row does not see, or the low half of a weight) times an
 // infinite value of another row's position is NaN.
 __device__ __forceinline__ void exact_row(const imh::PrefillAttention &a, size_t head_base, size_t qrow,
-                                                    int p_begin, int lim, int S, int split) {
+                                          int p_begin, int lim, int S, int split) {
     const int lane = threadIdx.x & 63;
     const _Float16 *q = a.q + qrow * kD;
     const _Float16 *k = reinterpret_cast<const _Float16 *>(a.k) + head_base * kD;
@@ -92,9 +92,9 @@ __device__ __forceinline__ void exact_row(const imh::PrefillAttention &a, size_t
         float nm = s;
         for (int st = 32; st >= 1; st >>= 1) nm = fmaxf(nm, __shfl_xor(nm, st));
         nm = fmaxf(nm, m);
-        const bool live = nm != -INFINITY;   // a row with no position yet keeps weight 0
+        // scores that are all -inf weigh 0, scores that are no numbers stay so
         const float corr = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - nm);
-        const float w = live && p0 + lane < lim ? __builtin_amdgcn_exp2f(s - nm) : 0.0f;
+        const float w = __builtin_amdgcn_exp2f(s - (nm == -INFINITY ? 0.0f : nm));
         m = nm;
         l = __builtin_fmaf(l, corr, w);
         o0 *= corr;
@@ -107,7 +107,10 @@ __device__ __forceinline__ void exact_row(const imh::PrefillAttention &a, size_t
         }
     }
     for (int st = 32; st >= 1; st >>= 1) l += __shfl_xor(l, st);
-    if (m == -INFINITY) o0 = o1 = 0.0f;
+    if (m == -INFINITY) {   // no position, or no score that is a number
+        if (l == 0.0f) o0 = o1 = 0.0f;
+        else m = 0.0f;
+    }
     if (S > 1) {
         const size_t pi = qrow * S + split;
         a.part_o[pi * kD + 2 * lane] = o0;

@@ -208,6 +208,7 @@ def test_row_tile_non_finite_values(dev, stream, nh, num_splits, aligned):
     cache.k.write(k)
     cache.v.write(v)
     q16 = np.random.default_rng(nh).standard_normal((batch, tokens, nh, D)).astype(np.float16)
+    q16[1, 60, 2, 7], q16[1, 61, 3, 8] = np.nan, np.inf   # these rows' scores are no numbers
     shift = 0 if aligned else 2
     qd, od = dev.buffer(q16.nbytes + 16), dev.buffer(q16.nbytes + 16)
     qd.write(q16, shift)
