@@ -415,7 +415,8 @@ int imh_encode_fp16_attention(imh_stream *stream, const imh_fp16_kv_cache *cache
     const uint32_t blocks = B * nkv * qblocks;
     const uint32_t L = seq_lens && seq_len == 0 ? cache->max_seq_len : seq_len;   // the bound of the lengths
     // The row tiles address a head's rows by 32-bit byte offsets: longer caches stay here.
-    if (token_count > 1 && L <= 0x7FFFFF && !(blocks <= 16 || (blocks <= 32 && L >= 8192)))
+    const bool tiles = token_count > 1 && L <= 0x7FFFFF;
+    if (tiles && !(blocks <= 16 || (blocks <= 32 && L >= 8192)))
         return prefill_attention(stream, cache, q, num_heads, gqa, token_count, seq_len, seq_lens, attn_scale, out,
                                  num_splits);
 
@@ -431,8 +432,13 @@ int imh_encode_fp16_attention(imh_stream *stream, const imh_fp16_kv_cache *cache
     const uint32_t S = std::max<uint32_t>(1, (L + split_len - 1) / split_len);
 
     const size_t nparts = (size_t)B * token_count * num_heads * S;
+    const size_t part_bytes = nparts * kD * 4 + nparts * 8 + 512;
     void *scr = nullptr;
-    rc = imh::stream_scratch(stream, 1, nparts * kD * 4 + nparts * 8 + 512, &scr);
+    // several tokens without room for the partials (a capture, or no memory): the row tiles, which need none
+    if (tiles && !imh::stream_scratch_optional(stream, 1, part_bytes, &scr))
+        return prefill_attention(stream, cache, q, num_heads, gqa, token_count, seq_len, seq_lens, attn_scale, out,
+                                 num_splits);
+    rc = imh::stream_scratch(stream, 1, part_bytes, &scr);
     if (rc) return rc;
     float *po = static_cast<float *>(scr);
     float *pm = po + nparts * kD;

@@ -253,3 +253,22 @@ def test_chunk_over_a_cache_past_32_bit_offsets(dev, stream):
     exact = 16384.0 * (seen - (ctx - ones)) / seen
     # f16 rounding of the result, 2^-11, and f32 sums of up to 2^17 equal terms per wave
     assert np.all(np.abs(got - exact[None, :, None, None]) <= 2.0 ** -9 * exact[None, :, None, None])
+
+
+@pytest.mark.parametrize("nh,tokens,bound", [(8, 16, 0), (8, 16, 8192), (32, 2, 0), (8, 40, 0)])
+def test_chunk_captured_without_scratch(dev, nh, tokens, bound):
+    """A capture of several tokens on a stream without room for any partials is accepted whichever
+    kernel the call's size asks for; replays equal the oracle."""
+    st = dev.stream()
+    cache = fill_cache(dev, st, 1, 8, 8192, 400, seed=201)
+    q16 = np.random.default_rng(202).standard_normal((1, tokens, nh, D)).astype(np.float16)
+    qd, od, sl = dev.upload(q16), dev.empty(q16.shape, np.float16), dev.upload(np.asarray([400], np.int32))
+    g = st.capture(lambda: ops.encode_fp16_attention(st, cache, qd, nh, bound, od, token_count=tokens,
+                                                     attn_scale=SCALE, seq_lens=sl))
+    ref = O.fp16_attention(q16, cache.k.read(), cache.v.read(), 8192, SCALE, nthreads=8,
+                           seq_lens=np.asarray([400], np.int32))
+    for _ in range(2):
+        st.zero(od)
+        g.launch()
+        st.sync()
+        assert_close(od.read(), ref, what=f"captured T={tokens} bound {bound}")
